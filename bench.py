@@ -48,10 +48,10 @@ sys.path.insert(0, ROOT)
 #   hpsi_nonloc_psi (the psi ratio at each quadrature point, its own kernel):
 #       Nao*42 per point
 # Executed matrix-core work of the quadrature kernel (k_nonloc_mma): every
-# group of up to four active pairs of a walker runs, for each 16-partner tile
-# and each step of four centres, 3 row tiles x naz table entries of one
-# 16x16x4 MFMA (2048 flop).  T = e-e-n terms (13 at nordc = 4), naz = the
-# non-zero A_kn table entries (12 at nordc = 4), Nc centres, Nao AOs.
+# group of up to four active pairs of a walker runs, for each 16-partner tile,
+# each 16-point tile and each step of four centres, one 16x16x4 MFMA (2048
+# flop) per coupled table entry.  T = e-e-n terms (13 at nordc = 4), coupled
+# entries C_kn with k, n >= 1 (3 at nordc = 4), Nc centres, Nao AOs.
 
 
 def flops_move_jastrow(ne, nc, nt, nao, nrad_total):
@@ -62,11 +62,11 @@ def flops_nonloc_point(ne, nc, nt, nao):
     return (ne - 1) * (nc * (4 * nt + 40) + 60) + nc * 40 + nao * 42
 
 
-def een_naz(nordc):
-    """Non-zero entries of the e-e-n tables A_kn (een_poly.hpp): term (k, l, m)
-    fills A[k][m] and A[k][l + m]."""
+def een_ncoupled(nordc):
+    """Entries C_kn (k, n >= 1) of the split e-e-n polynomial (een_poly.hpp):
+    term (k, l, m) with k, m >= 1 fills C[k][m] and C[k][l + m]."""
     from champ_amd import system as S
-    return len({(k, m) for k, l, m in S.een_terms(nordc)} | {(k, l + m) for k, l, m in S.een_terms(nordc)})
+    return len({(k, n) for k, l, m in S.een_terms(nordc) if k >= 1 and m >= 1 for n in (m, l + m)})
 
 
 def mfma_flops_nonloc(sy, nxq):
@@ -74,9 +74,9 @@ def mfma_flops_nonloc(sy, nxq):
     pair counts (nxquad / nquad per walker)."""
     nq = max(1, len(sy.wq))
     pairs = np.asarray(nxq, dtype=np.int64) // nq
-    groups = int(np.sum((pairs + 3) // 4))
-    per_group = -(-sy.nelec // 16) * -(-sy.ncent // 4) * 3 * een_naz(sy.nordc) * 2048
-    return float(groups) * per_group
+    row_tiles = int(np.sum((pairs // 4) * (-(-4 * nq // 16)) + -(-(pairs % 4) * nq // 16)))
+    per_tile = -(-sy.nelec // 16) * -(-sy.ncent // 4) * een_ncoupled(sy.nordc) * 2048
+    return float(row_tiles) * per_tile
 
 
 def run_path(sy, W, precision, args, label):
@@ -231,8 +231,8 @@ def per_kernel(sy, W, kt, nxq, path, acc):
                          "reference count Ne(Ne-1)/2 Nc (54T+80) per walker", False),
         "hpsi_mo_gemm": (2.0 * wchunk * ne * 5 * no * nb, "fp64-mfma", "TFLOP/s", "2 (5 Ne W_chunk) norb Nao", True),
         "hpsi_slater_lu": (wchunk * 2 * 2.0 * ns ** 3, "fp64-valu", "TFLOP/s", "2 Nsigma^3 per spin matrix", True),
-        "hpsi_nonloc": (mfma_flops_nonloc(sy, nxq), mfma, "TFLOP/s", "executed 16x16x4 MFMA flop (groups x "
-                        "partner tiles x centre quads x 3 row tiles x naz)", True),
+        "hpsi_nonloc": (mfma_flops_nonloc(sy, nxq), mfma, "TFLOP/s", "executed 16x16x4 MFMA flop (point tiles x "
+                        "partner tiles x centre quads x coupled entries)", True),
         "hpsi_nonloc_psi": (float(np.sum(nxq)) * nb * 42, "fp64-valu", "TFLOP/s",
                             "reference count Nao*42 per quadrature point (AO values at the point, dot with W)", False),
     }
@@ -272,7 +272,7 @@ def roofline(sy, W, kt, nxq, path, acc):
         r["quadrature_points_per_launch"] = int(npts)
         r["work_equivalent"] = {
             "achieved": round(ref / t / 1e12, 3), "unit": "TFLOP/s",
-            "basis": "reference per-term count per point x points; the factorised kernel executes ~7x fewer "
+            "basis": "reference per-term count per point x points; the factorised kernel executes far fewer "
                      "operations, so this rate is not a utilisation"}
     return r
 

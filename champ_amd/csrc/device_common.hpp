@@ -19,6 +19,81 @@ __device__ __forceinline__ T wave_sum(T v)
     return v;
 }
 
+// v of the lane that the DPP control word names, by a register move of the
+// vector pipe (__shfl_xor goes through LDS)
+template <int CTRL>
+__device__ __forceinline__ double dpp_mov(double v)
+{
+    union { double d; int i[2]; } u, r;
+    u.d = v;
+    r.i[0] = __builtin_amdgcn_mov_dpp(u.i[0], CTRL, 0xf, 0xf, true);
+    r.i[1] = __builtin_amdgcn_mov_dpp(u.i[1], CTRL, 0xf, 0xf, true);
+    return r.d;
+}
+// sum over the 16 lanes of a row (lanes of equal lane / 16), in every lane:
+// pairs, quads, then the mirrored halves, whose quads hold equal values
+__device__ __forceinline__ double row16_sum(double v)
+{
+    v += dpp_mov<0xB1>(v);   // quad_perm 1 0 3 2
+    v += dpp_mov<0x4E>(v);   // quad_perm 2 3 0 1
+    v += dpp_mov<0x141>(v);  // row_half_mirror
+    v += dpp_mov<0x140>(v);  // row_mirror
+    return v;
+}
+
+// ---------------------------------------------------------- FP64 functions
+// Square root, exponential and quotient for the inner loops, where operands
+// are ordinary distances: without the denormal scaling and the range checks
+// of the general functions, and with the polynomial of the exponential in
+// Estrin's form, which is half as long a chain as Horner's.  Newton and
+// Goldschmidt steps from the hardware estimates bring each to within an ulp
+// or two of the exact value (tests/cpu_emu/fastmath_check.cpp); 0 and infinity
+// give what the general functions give, NaN stays NaN.
+__device__ __forceinline__ double sqrt_inner(double x)
+{
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    const double d = __builtin_fma(-h, g, 0.5);
+    g = __builtin_fma(g, d, g);
+    h = __builtin_fma(h, d, h);
+    g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+    g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+    return (x == 0.0 || x == __builtin_inf()) ? x : g;
+}
+// exp(x) for x <= 0: x = n ln 2 + f, the Taylor polynomial of degree 13 on
+// |f| <= ln 2 / 2 (remainder 4e-18)
+__device__ __forceinline__ double exp_neg(double x)
+{
+    const double xc = x < -800.0 ? -800.0 : x;
+    const double n = __builtin_rint(xc * 1.4426950408889634);
+    double f = __builtin_fma(n, -6.93147180369123816490e-01, xc);
+    f = __builtin_fma(n, -1.90821492927058770002e-10, f);
+    const double f2 = f * f, f4 = f2 * f2;
+    const double p2 = __builtin_fma(f, 1.0 / 6, 0.5);
+    const double p4 = __builtin_fma(f, 1.0 / 120, 1.0 / 24);
+    const double p6 = __builtin_fma(f, 1.0 / 5040, 1.0 / 720);
+    const double p8 = __builtin_fma(f, 1.0 / 362880, 1.0 / 40320);
+    const double p10 = __builtin_fma(f, 1.0 / 39916800, 1.0 / 3628800);
+    const double p12 = __builtin_fma(f, 1.0 / 6227020800.0, 1.0 / 479001600);
+    const double q4 = __builtin_fma(f2, p6, p4), q8 = __builtin_fma(f2, p10, p8);
+    const double r4 = __builtin_fma(f4, __builtin_fma(f4, p12, q8), q4);
+    // 1 + f + f2 (p2 + f2 r4), the small part added last
+    const double t = __builtin_fma(f2, __builtin_fma(f2, r4, p2), f);
+    return ldexp(1.0 + t, (int)n);
+}
+__device__ __forceinline__ double div_inner(double a, double b)
+{
+    double y = __builtin_amdgcn_rcp(b);
+    y = __builtin_fma(__builtin_fma(-b, y, 1.0), y, y);
+    y = __builtin_fma(__builtin_fma(-b, y, 1.0), y, y);
+    const double q = a * y;
+    return __builtin_fma(__builtin_fma(-b, q, a), y, q);
+}
+// the FP32 forms are the general functions
+__device__ __forceinline__ float sqrt_inner(float x) { return sqrtf(x); }
+__device__ __forceinline__ float exp_neg(float x) { return expf(x); }
+__device__ __forceinline__ float div_inner(float a, float b) { return a / b; }
+
 // --------------------------------------------------------------- xoshiro256**
 // Blackman & Vigna (2018), bound by CHAMP through random.f90:3-55.
 __device__ __forceinline__ uint64_t rotl64(uint64_t x, int k) { return (x << k) | (x >> (64 - k)); }

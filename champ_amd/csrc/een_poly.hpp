@@ -185,4 +185,75 @@ __device__ __forceinline__ EenOut<T> een_eval_tab(const T *tab, T u, T y)
     return o;
 }
 
+// ------------------------------------------------------------------------
+// The same polynomial split by what each part couples.  A term with m = 0 is
+// c u^k (x^l + y^l): it depends on one electron-centre distance at a time, so
+// summed over the centres it is u^k (X_k + Y_k) with one number per electron
+// and power (k = 1 .. N - 1).  Only the terms with m >= 1 couple x and y:
+//     sum_{k, n >= 1} C_kn(y) x^n u^k   (k = 0 .. N - 2),
+// and those with k = 0 do not hold u, so that a sum over the partners needs
+// sum_j C_0n(y_j) only.  At N = 4 three coupled entries (k >= 1) remain of
+// the twelve of EenTable, at N = 5 six of eighteen.
+template <int N>
+struct EenSplit {
+    int idx[N + 1][N + 1];  // packed position of C_kn, k >= 1, -1 where zero
+    int nc;                 // number of them
+    int kmax;               // highest coupled power of u (N - 2), 0 if none with k >= 1
+    int nmax;               // highest power of x among them
+    constexpr EenSplit() : idx{}, nc(0), kmax(0), nmax(0)
+    {
+        constexpr EenTable<N> ET{};
+        bool nz[N + 1][N + 1] = {};
+        for (int t = 0; t < ET.n; t++)
+            if (ET.m[t] >= 1) {
+                nz[ET.k[t]][ET.m[t]] = true;
+                nz[ET.k[t]][ET.l[t] + ET.m[t]] = true;
+            }
+        for (int kk = 0; kk <= N; kk++)
+            for (int nn = 0; nn <= N; nn++) {
+                idx[kk][nn] = (kk >= 1 && nz[kk][nn]) ? nc++ : -1;
+                if (idx[kk][nn] >= 0) {
+                    if (kk > kmax) kmax = kk;
+                    if (nn > nmax) nmax = nn;
+                }
+            }
+    }
+};
+// numbers per electron of the uncoupled part, and of C_0n (both N - 1)
+template <int N>
+constexpr int een_nsep() { return N > 1 ? N - 1 : 0; }
+
+// C_kn(y) of one (k, n); yp: the powers of y
+template <int N, typename T>
+__device__ __forceinline__ T een_coupled(const double *c, const T *yp, int k, int n)
+{
+    constexpr EenTable<N> ET{};
+    T v = T(0);
+#pragma unroll
+    for (int t = 0; t < ET.n; t++) {
+        if (ET.m[t] < 1 || ET.k[t] != k) continue;
+        if (ET.m[t] == n) v += (T)c[t] * yp[ET.l[t] + ET.m[t]];
+        if (ET.l[t] + ET.m[t] == n) v += (T)c[t] * yp[ET.m[t]];
+    }
+    return v;
+}
+
+template <int N, typename T>
+__device__ __forceinline__ void een_powers(T y, T *yp)
+{
+    yp[0] = T(1);
+#pragma unroll
+    for (int p = 1; p <= N; p++) yp[p] = p == 1 ? y : y * yp[p - 1];
+}
+
+// s[k - 1] += sum over the uncoupled terms of power k of c_t y^l
+template <int N, typename T>
+__device__ __forceinline__ void een_uncoupled(const double *c, const T *yp, T *s)
+{
+    constexpr EenTable<N> ET{};
+#pragma unroll
+    for (int t = 0; t < ET.n; t++)
+        if (ET.m[t] == 0) s[ET.k[t] - 1] += (T)c[t] * yp[ET.l[t]];
+}
+
 }  // namespace champ

@@ -392,6 +392,8 @@ extern "C" int champ_gpu_init(champ_ctx **ctxp, const champ_system_t *s, int32_t
         TRY(dalloc(&c->pair_val, (size_t)W * c->pair_cap));
         TRY(dalloc(&c->pair_psi, (size_t)W * c->pair_cap * std::max(c->NQ, 1)));
         TRY(dalloc(&c->rrT, (size_t)W * NE * NC));
+        const size_t nsep = std::max(1, s->nordc - 1);
+        TRY(dalloc(&c->een_ys, (size_t)W * nsep * NE)); TRY(dalloc(&c->een_t0, (size_t)W * nsep * NC));
     }
     TRY(dalloc(&c->pair_count, W)); TRY(dalloc(&c->pair_off, (size_t)W + 1)); TRY(dalloc(&c->pair_total, 2));
     TRY(dalloc(&c->grp_off, (size_t)W + 1));
@@ -442,7 +444,7 @@ extern "C" int champ_gpu_free(champ_ctx *c)
                     c->esum_dev, c->aoall, c->orball, c->wmat, c->pair_count, c->pair_off, c->pair_total, c->grp_off,
                     c->pair_e, c->pair_c, c->pair_vps, c->pair_val, c->pair_psi, c->rrT, c->nxquad, c->ri_cent, c->ri_type,
                     c->ri_rad, c->ri_rmax, c->ao_ri, c->gref, c->lu_ws, c->m6rec, c->ri_perm,
-                    c->ri_aoff, c->ri_aol, c->enp, c->gemm_tmp};
+                    c->ri_aoff, c->ri_aol, c->enp, c->gemm_tmp, c->een_ys, c->een_t0};
     for (void *p : ptrs) if (p) hipFree(p);
     md_free(c);
     dmc_free(c);
@@ -857,6 +859,7 @@ extern "C" int champ_gpu_autotune(champ_ctx *c, int32_t *choices)
         for (int kind : {0, 1}) {
             c->tune_nonloc = kind;
             float ms = 0;
+            if ((rc = launch_hpsi_impl(c, 0))) break;  // each form's own inputs (rrT or the split sums)
             if ((rc = time_launch(c, tune_nonloc, 3, &ms))) break;
             if (ms < best) { best = ms; pick = kind; }
         }

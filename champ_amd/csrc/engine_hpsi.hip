@@ -575,6 +575,10 @@ __device__ double gauss_pot(const EcpParams &ep, int ict, int l, double r)
 // getvps_gauss + local part of nonloc_pot + active (electron, centre) list
 // in the order of nonloc.f90:126-186.  One block per walker, threads over
 // electrons, deterministic order by a block-wide scan.
+// NS > 1: also the split e-e-n sums of order NS that the matrix-core
+// quadrature reads: per electron Y_k = sum_b sum_(m = 0) c_t y_jb^l, per centre
+// sum_j C_0n(y_jb) (one more pass over r_en, in cache).
+template <int NS>
 __global__ void __launch_bounds__(256) k_hpsi_vps(HArgs a)
 {
     __shared__ int cnt[1024];
@@ -626,10 +630,38 @@ __global__ void __launch_bounds__(256) k_hpsi_vps(HArgs a)
             off++;
         }
     }
-    // rr_en with the centre index innermost for the quadrature kernel
     const double *rrw = a.rr_en + (size_t)w * NC * NE;
-    double *rrt = a.rrT + (size_t)w * NE * NC;
-    for (int t = tid; t < NE * NC; t += bd) rrt[t] = rrw[(size_t)(t % NC) * NE + t / NC];
+    if (a.rrt) {  // rr_en with the centre index innermost for the vector-pipe quadrature
+        double *rrt = a.rrT + (size_t)w * NE * NC;
+        for (int t = tid; t < NE * NC; t += bd) rrt[t] = rrw[(size_t)(t % NC) * NE + t / NC];
+    }
+    if constexpr (NS > 1) {
+        constexpr int NP = een_nsep<NS>();
+        const JasParams &jp = *a.jas;
+        const int lane = tid % WAVE, wv = tid / WAVE, nwv = bd / WAVE;
+        for (int e = tid; e < NE; e += bd) {
+            double s[NP] = {0}, yp[NS + 1];
+            for (int c = 0; c < NC; c++) {
+                een_powers<NS>(1.0 - jp.kap * rrw[(size_t)c * NE + e], yp);
+                een_uncoupled<NS>(jp.c[a.iwctype[c]], yp, s);
+            }
+            for (int k = 0; k < NP; k++) a.een_ys[((size_t)w * NP + k) * NE + e] = s[k];
+        }
+        for (int c = wv; c < NC; c += nwv) {
+            const double *ct = jp.c[a.iwctype[c]];
+            double s[NP] = {0}, yp[NS + 1];
+            for (int e = lane; e < NE; e += WAVE) {
+                een_powers<NS>(1.0 - jp.kap * rrw[(size_t)c * NE + e], yp);
+#pragma unroll
+                for (int n = 1; n <= NP; n++) s[n - 1] += een_coupled<NS>(ct, yp, 0, n);
+            }
+#pragma unroll
+            for (int n = 0; n < NP; n++) {
+                const double v = wave_sum(s[n]);
+                if (lane == 0) a.een_t0[((size_t)w * NP + n) * NC + c] = v;
+            }
+        }
+    }
     const double pes = block_sum(pe, red);
     if (tid == 0) a.pe_local[w] = pes;
 }
@@ -939,7 +971,15 @@ int launch_hpsi_impl(champ_ctx *c, int accumulate)
     if (c->nloc > 0) {
         // vps and the active-pair list, their offsets, the coefficient rows
         tbegin(c, K_HPSI_ECP, &slot);
-        hipLaunchKernelGGL(k_hpsi_vps, dim3(c->W), dim3(256), 0, c->stream, a);
+        const bool mma = nonloc_on_matrix_cores(c);
+        a.rrt = !mma;
+        switch (mma ? c->hjas.nordc : 0) {
+        case 2: hipLaunchKernelGGL(k_hpsi_vps<2>, dim3(c->W), dim3(256), 0, c->stream, a); break;
+        case 3: hipLaunchKernelGGL(k_hpsi_vps<3>, dim3(c->W), dim3(256), 0, c->stream, a); break;
+        case 4: hipLaunchKernelGGL(k_hpsi_vps<4>, dim3(c->W), dim3(256), 0, c->stream, a); break;
+        case 5: hipLaunchKernelGGL(k_hpsi_vps<5>, dim3(c->W), dim3(256), 0, c->stream, a); break;
+        default: hipLaunchKernelGGL(k_hpsi_vps<0>, dim3(c->W), dim3(256), 0, c->stream, a); break;
+        }
         HIPCHECK(hipGetLastError());
         hipLaunchKernelGGL(k_pair_scan, dim3(1), dim3(1024), 0, c->stream, c->W, c->pair_count, c->pair_off, c->pair_total, 1);
         HIPCHECK(hipGetLastError());

@@ -163,6 +163,9 @@ struct champ_ctx {
     int tstore = 0;                            // hpsi keeps each quadrature point's t_vpsp in pair_psi (T-moves)
     double *rrT = nullptr;                     // [W][NE][NC] rr_en with the centre innermost
     int *nxquad = nullptr;                     // [W]
+    // split e-e-n sums of the matrix-core quadrature: Y_k [W][nordc-1][NE] and
+    // sum_j C_0n [W][nordc-1][NC]
+    double *een_ys = nullptr, *een_t0 = nullptr;
 
     // ---- multideterminant (ndet > 1): excitation tables per spin and state
     int md = 0, md_ndet = 0, md_NV = 0, md_NU = 0, md_nu[2] = {0, 0}, md_nv[2] = {0, 0};

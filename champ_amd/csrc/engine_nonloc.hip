@@ -300,28 +300,35 @@ __global__ void __launch_bounds__(NL_THREADS) CHAMP_WAVES_PER_EU(CHAMP_NL_WPE) k
 }
 
 // ------------------------------------------------------------------------
-// Matrix-core form of the quadrature's e-e-n sum.  By the x <-> y symmetry of
-// the polynomial, P(u, x, y) = sum_k u^k sum_n A_kn(y) x^n with the tables
-// A_kn of the partner's distance y (een_poly.hpp).  For the points q of a
-// group of pairs and the partners j of one walker,
-//   M_k[q][j] = sum_{(b, n)} x_qb^n A_kn(y_jb)          (K = centres x powers)
-// is a product of a (points x K) matrix of powers by a (K x partners) matrix
-// of partner tables, and the e-e-n sum of point q is
-//   sum_{j != i} sum_k u_qj^k M_k[q][j].
+// Matrix-core form of the quadrature's e-e-n sum.  With the split of
+// een_poly.hpp the sum of point q (electron i, switched distances x_qb) over
+// its partners j is
+//   sum_{j != i} sum_{k >= 1} u_qj^k (M_k[q][j] + X_k[q] + Y_k[j])
+//     + sum_b sum_n x_qb^n (sum_j C_0n(y_jb) - C_0n(y_ib)),
+//   M_k[q][j] = sum_{(b, n)} x_qb^n C_kn(y_jb).
+// Only M_k is a product of matrices, a (points x centres*powers) by a
+// (centres*powers x partners) one with nc entries per centre (3 at N = 4);
+// X_k is formed once per point, Y_k and sum_j C_0n once per walker
+// (k_hpsi_vps).  Against a product with all twelve entries of A_kn this runs a
+// quarter of the matrix instructions.
 // A block takes MMA_GP active pairs of one walker (MMA_GP * NQ <= 48 points:
-// three 16-row tiles).  Items (16 partners) are dealt to the four waves.  An
+// three 16-row tiles).  Items (16 partners x 16 points) are dealt to the four
+// waves in contiguous runs; up to three items of one partner tile run
+// together, so that a lane builds the partner's entries once for them.  An
 // item walks the centres four at a time: the four K-slots of an MFMA are four
-// centres at one table entry (k, n), so a lane builds all table entries of
-// its (centre, partner) once and feeds, for each row tile, one
-// v_mfma_f64_16x16x4f64 per entry into the accumulator of row k (lane l
-// supplies A[l % 16][l / 16] and B[l / 16][l % 16]; element r of the
-// accumulator holds D[4 r + l / 16][l % 16]).  The partner distances are read
-// from rr_en, partners innermost, so the 16 lanes of a slot load one line.
-// The epilogue recomputes u_qj for its 4 x 1 (point, partner) entries and adds
-// sum_k u^k M_k to per-lane point sums.  The e-e and e-n sums and the psi
-// ratio are computed as in k_nonloc.
+// centres at one entry (k, n) (lane l supplies A[l % 16][l / 16] and
+// B[l / 16][l % 16]; element r of the accumulator holds the row of Mma::row).
+// The partner distances are read from rr_en, partners innermost, so the 16
+// lanes of a slot load one line.  The epilogue forms u_qj and the e-e term of
+// its 4 x 1 (point, partner) entries and adds to sums in registers, reduced
+// over the lanes once per group.
+// Bound: the epilogue (square root, exponential and Pade division per
+// (point, partner)) on the vector pipe, with the matrix cores beside it; three
+// waves per SIMD (168 registers) hide more of both than two.
+// Measured (160 electrons, 40 centres, 4096 walkers, about 1e7 points): 40.7 ms
+// with all entries in the product, 17.1 ms now; FP32 28.8 and 13.1 ms.
 constexpr int MMA_GP = NL_GROUP, MMA_MT = 3, MMA_MP = 16 * MMA_MT, MMA_THREADS = 256, MMA_WAVES = MMA_THREADS / WAVE;
-constexpr int MMA_TG = MMA_THREADS / MMA_MP;  // thread groups over (point, partner) in the point phase
+constexpr int MMA_TG = MMA_THREADS / MMA_MP;  // thread groups over (point, centre) in the point phase
 
 // accumulator type and instruction per arithmetic type; row of accumulator
 // element r in lane slot sl = l / 16 (measured on gfx950 with one-hot
@@ -340,123 +347,177 @@ template <> struct Mma<float> {
     static __device__ __forceinline__ int row(int r, int sl) { return 4 * sl + r; }
 };
 
-// with_ee: the item also adds the e-e terms b(u_qj) of its (point, partner)
-// entries (the first of the two halves of a split tile, or a whole tile)
-template <int N, typename T>
-__device__ __forceinline__ void mma_item(const HArgs &a, int w, int j0, int c_lo, int c_hi, int npts,
-                                         const double *XP, const T *XQ, const int *IPT, double *swv, bool with_ee,
-                                         const JasParams &jp, const int *sT)
+// The e-e term minus its asymptote of the epilogue, per spin class (0 unlike,
+// 1 like) in a block's LDS: psi = p0 u / (1 + p1 u) - p2 + u^2 (p3 + u (p4 + ...)),
+// the coefficients past nordb zero.  The float form is (u - U)(p0 / (1 + p1 u)
+// + p2 + u (p3 + ...)), pade_minus_asym with its powers of the asymptote U
+// multiplied out (all of one sign pattern with the coefficients: nothing new
+// cancels).
+constexpr int EE_NP = CHAMP_NORDP + 1;
+template <typename T>
+__device__ __forceinline__ void ee_table(const JasParams &jp, T *tab)
 {
-    constexpr EenTable<N> ET{};
-    constexpr int NA = een_naz<N>(), KR = ET.kmax + 1;
+    for (int t = threadIdx.x; t < 2 * EE_NP; t += MMA_THREADS) {
+        const int like = t / EE_NP, o = t % EE_NP;
+        const double *b = jp.b[(like && jp.nspin2b == 2) ? 1 : 0];
+        const double s0 = (like && jp.nspin2b == 1 && jp.nocuspb == 0) ? 0.5 : 1.0, U = jp.asymp_r;
+        double v;
+        if constexpr (sizeof(T) == sizeof(float)) {
+            if (o == 0) v = s0 * b[0] / (1.0 + b[1] * U);
+            else if (o == 1) v = b[1];
+            else {  // coefficient of u^(o - 2): sum over the orders q >= o of b_q U^(q - 1 - (o - 2))
+                v = 0.0;
+                for (int q = jp.nordb; q >= 2 && q >= o - 1; q--) v += b[q] * powi(U, q - o + 1);
+            }
+        } else {
+            v = o == 0 ? s0 * b[0] : o == 1 ? b[1] : o == 2 ? jp.jb[like] : (o - 1 <= jp.nordb ? b[o - 1] : 0.0);
+        }
+        tab[t] = (T)v;
+    }
+}
+
+template <typename T>
+__device__ __forceinline__ T ee_from_table(const T *p, T rr, T u, double asymp_r)
+{
+    const T pade = div_inner(p[0], T(1) + p[1] * rr);
+    if constexpr (sizeof(T) == sizeof(float)) {
+        T g = p[EE_NP - 1];
+#pragma unroll
+        for (int o = EE_NP - 2; o >= 2; o--) g = g * rr + p[o];
+        return asym_offset<T>(asymp_r, u) * (pade + g);
+    } else {
+        T g = p[EE_NP - 1];
+#pragma unroll
+        for (int o = EE_NP - 2; o >= 3; o--) g = g * rr + p[o];
+        return rr * pade - p[2] + g * (rr * rr);
+    }
+}
+
+#ifndef CHAMP_MMA_ILP
+#define CHAMP_MMA_ILP 1
+#endif
+
+// MTN row tiles from mt0 of the partner tile at j0, added to psum[row tile][r]
+template <int N, typename T, int MTN>
+__device__ __forceinline__ void mma_item(const HArgs &a, int w, int j0, int mt0, int npts, const double *XP, const T *XQ,
+                                         const double *XK, const int *IPT, double (&psum)[MMA_MT][4],
+                                         const JasParams &jp, const int *sT, const T *EE)
+{
+    constexpr EenSplit<N> ES{};
+    constexpr int NE_ = ES.nc > 0 ? ES.nc : 1, KC = ES.kmax > 0 ? ES.kmax : 1, NP = een_nsep<N>();
     typedef typename Mma<T>::acc Acc;
     const int lane = threadIdx.x % WAVE, sl = lane / 16, ln = lane % 16;
     const int NC = a.NC, NE = a.NE;
     const double kap = jp.kap;
     const int j = j0 + ln;
     const bool jv = j < NE;
-    const double *rrw = a.rr_en + (size_t)w * NC * NE;
-    Acc acc[MMA_MT][KR];
+    const int jq = jv ? j : 0;
+    Acc acc[MTN][KC];
 #pragma unroll
-    for (int mt = 0; mt < MMA_MT; mt++)
+    for (int mt = 0; mt < MTN; mt++)
 #pragma unroll
-        for (int k = 0; k < KR; k++) acc[mt][k] = Mma<T>::zero();
-    // partner distances two centre steps ahead
-    double ynext = (jv && c_lo + sl < c_hi) ? rrw[(size_t)(c_lo + sl) * NE + j] : 0.0;
-    double ynext2 = (jv && c_lo + sl + 4 < c_hi) ? rrw[(size_t)(c_lo + sl + 4) * NE + j] : 0.0;
-    for (int b0 = c_lo; b0 < c_hi; b0 += 4) {
-        const int b = b0 + sl;
-        const bool bv = b < c_hi;
-        const double rrb = ynext;
-        ynext = ynext2;
-        if (b + 8 < c_hi && jv) ynext2 = rrw[(size_t)(b + 8) * NE + j];
-        // the partner's table entries at centre b: built once, used by every row tile
-        T tab[NA];
-        een_tables<N, 0, T>(jp.c[bv ? sT[b] : 0], (T)(1.0 - kap * rrb), tab);
-        if (!(bv && jv)) {
+        for (int k = 0; k < KC; k++) acc[mt][k] = Mma<T>::zero();
+    if constexpr (ES.nc > 0) {
+        const double *rrw = a.rr_en + (size_t)w * NC * NE + jq;
+        // partner distances two centre steps ahead
+        double ynext = rrw[(size_t)min(sl, NC - 1) * NE], ynext2 = rrw[(size_t)min(sl + 4, NC - 1) * NE];
+        for (int b0 = 0; b0 < NC; b0 += 4) {
+            const int b = b0 + sl;
+            const bool bv = b < NC;
+            const double rrb = ynext;
+            ynext = ynext2;
+            if (b0 + 8 < NC) ynext2 = rrw[(size_t)min(b + 8, NC - 1) * NE];
+            // the partner's entries at centre b, used by every row tile; every
+            // coupled entry holds a positive power of y, so y = 0 clears the
+            // lanes past the partners or the centres (XQ is padded with zeros)
+            T yp[N + 1], tab[NE_];
+            een_powers<N, T>((bv && jv) ? (T)(1.0 - kap * rrb) : T(0), yp);
+            const double *ct = jp.c[bv ? sT[b] : 0];
 #pragma unroll
-            for (int e = 0; e < NA; e++) tab[e] = T(0);
+            for (int k = 1; k <= KC; k++)
+#pragma unroll
+                for (int n = 1; n <= ES.nmax; n++)
+                    if (ES.idx[k][n] >= 0) tab[ES.idx[k][n]] = een_coupled<N, T>(ct, yp, k, n);
+            T xp[MTN][N + 1];
+#pragma unroll
+            for (int mt = 0; mt < MTN; mt++) een_powers<N, T>(XQ[(size_t)b * MMA_MP + (mt0 + mt) * 16 + ln], xp[mt]);
+            // consecutive MFMAs go to different accumulators (row tile, power of
+            // u), so none waits for the previous one's result
+#pragma unroll
+            for (int n = 1; n <= ES.nmax; n++)
+#pragma unroll
+                for (int k = 1; k <= KC; k++) {
+                    if (ES.idx[k][n] < 0) continue;
+#pragma unroll
+                    for (int mt = 0; mt < MTN; mt++)
+                        acc[mt][k - 1] = Mma<T>::op(xp[mt][n], tab[ES.idx[k][n]], acc[mt][k - 1]);
+                }
         }
-        T xp[MMA_MT][N + 1];
-#pragma unroll
-        for (int mt = 0; mt < MMA_MT; mt++) {
-            const int pta = mt * 16 + ln;
-            const bool live_a = bv && pta < npts;
-            const T x = live_a ? XQ[(size_t)b * MMA_MP + pta] : T(0);
-            xp[mt][0] = live_a ? T(1) : T(0);
-#pragma unroll
-            for (int p = 1; p <= N; p++) xp[mt][p] = xp[mt][p - 1] * x;
-        }
-        // consecutive MFMAs go to different accumulators (row tile, power of
-        // u), so none waits for the previous one's result
-#pragma unroll
-        for (int n = 0; n <= N; n++)
-#pragma unroll
-            for (int k = 0; k < KR; k++) {
-                const int e = ET.idx[k][n];
-                if (e < 0) continue;
-#pragma unroll
-                for (int mt = 0; mt < MMA_MT; mt++) acc[mt][k] = Mma<T>::op(xp[mt][n], tab[e], acc[mt][k]);
-            }
     }
     const double *xw = a.xT + (size_t)w * 3 * NE;
-    const double xj = jv ? xw[j] : 0.0, yj = jv ? xw[NE + j] : 0.0, zj = jv ? xw[2 * NE + j] : 0.0;
+    const double xj = xw[jq], yj = xw[NE + jq], zj = xw[2 * NE + jq];
+    double ys[NP];
 #pragma unroll
-    for (int mt = 0; mt < MMA_MT; mt++)
+    for (int k = 0; k < NP; k++) ys[k] = a.een_ys[((size_t)w * NP + k) * NE + jq];
+#pragma unroll
+    for (int mt = 0; mt < MTN; mt++)
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-            const int pt = mt * 16 + Mma<T>::row(r, sl);
-            double v = 0.0;
-            if (jv && pt < npts && j != IPT[pt]) {
-                // the switched e-e distance as the point phase forms it
-                const T d0 = (T)(xj - XP[3 * pt]), d1 = (T)(yj - XP[3 * pt + 1]), d2 = (T)(zj - XP[3 * pt + 2]);
-                T r2 = 0;
-                r2 = r2 + d0 * d0; r2 = r2 + d1 * d1; r2 = r2 + d2 * d2;
-                const T rjq = sqrt(r2);
-                const T rr = scale_r<T>((T)kap, rjq);
-                const T u = switched_from<T>(kap, rjq, rr);
-                T pv2 = acc[mt][KR - 1][r];
+            // every lane runs the entry (a branch would keep the entries from
+            // overlapping); the ones that do not count are dropped at the end
+            const int pt = (mt0 + mt) * 16 + Mma<T>::row(r, sl);
+            const int ipt = IPT[pt];  // -1 past the group's points
+            const T d0 = (T)(xj - XP[3 * pt]), d1 = (T)(yj - XP[3 * pt + 1]), d2 = (T)(zj - XP[3 * pt + 2]);
+            T r2 = 0;
+            r2 = r2 + d0 * d0; r2 = r2 + d1 * d1; r2 = r2 + d2 * d2;
+            // the switched distance u = exp(-kap r) and the scaled one (1 - u) / kap
+            const T u = exp_neg((T)(-kap * (double)sqrt_inner(r2)));
+            const T rr = (T(1) - u) * (T)jp.asymp_r;
+            T pv = T(0);
 #pragma unroll
-                for (int k = KR - 2; k >= 0; k--) pv2 = pv2 * u + acc[mt][k][r];
-                v = (double)pv2;
-                if (with_ee) v += (double)ee_term<T>(jp, a.NUP, IPT[pt], j, rr, u);
+            for (int k = NP; k >= 1; k--) {
+                const T m = (T)(XK[(k - 1) * MMA_MP + pt] + ys[k - 1]);
+                pv = pv * u + ((k <= ES.kmax) ? (T)(m + acc[mt][k <= KC ? k - 1 : 0][r]) : m);
             }
-            // sum over the 16 partners (lanes of equal l / 16) into the wave's point slot
-            v += __shfl_xor(v, 1, WAVE); v += __shfl_xor(v, 2, WAVE);
-            v += __shfl_xor(v, 4, WAVE); v += __shfl_xor(v, 8, WAVE);
-            if (ln == 0) swv[pt] += v;
+            const bool like = (ipt < a.NUP) == (jq < a.NUP);
+            const double e = (double)(pv * u) + (double)ee_from_table<T>(EE + (like ? EE_NP : 0), rr, u, jp.asymp_r);
+            const double v = (jv && ipt >= 0 && j != ipt) ? e : 0.0;
+            if constexpr (MTN == MMA_MT) {
+                psum[mt][r] += v;
+            } else {
+#pragma unroll
+                for (int t = 0; t < MMA_MT; t++)
+                    if (t == mt0 + mt) psum[t][r] += v;
+            }
+            // CHAMP_MMA_ILP entries overlap; more would cost a wave of occupancy in registers
+            if (r % CHAMP_MMA_ILP == CHAMP_MMA_ILP - 1) __builtin_amdgcn_sched_barrier(0);
         }
 }
 
-// psi-ratio phase: lanes over (point, radial-instance slot), MMA_PS slots
-constexpr int MMA_PS = MMA_THREADS / MMA_MP;
-static_assert(MMA_PS * MMA_MP <= 2 * MMA_TG * MMA_MP, "psi-ratio partials fit the point-phase partials");
-
-// LDS of k_nonloc_mma in doubles: XP, SP, TG partials (reused for the
-// psi-ratio partials), SW, FI, IPT/PI (as doubles), XQ (tsize bytes per
-// entry), the point-centre distances (double) and grid indices (int), then
-// the radial instances in slot order (8 ints and the cut radius each) and the
-// AOs in slot order (slm code and AO index)
-__host__ __device__ __forceinline__ size_t mma_lds_doubles(int NC, int NB, int NRI, int tsize)
+// LDS of k_nonloc_mma in doubles: XP, SP (e-n and uncoupled sums, e-e and
+// e-e-n), partials of the point phase, SW, FI, IPT/PI (as doubles), XK, the
+// pairs' k = 0 weights and XQ (tsize bytes per entry, centres padded to four)
+__host__ __device__ __forceinline__ size_t mma_lds_doubles(int NC, int nordc, int tsize)
 {
-    return 3 * MMA_MP + 3 * MMA_MP + 2 * MMA_TG * MMA_MP + MMA_WAVES * MMA_MP + MMA_GP + MMA_MP + 4 * MMA_GP +
-           ((size_t)NC * MMA_MP * tsize + 7) / 8 + (size_t)NC * MMA_MP + ((size_t)NC * MMA_MP * 4 + 7) / 8 +
-           (size_t)NRI * 4 + (size_t)NRI + (size_t)NB;
+    const int np = nordc > 1 ? nordc - 1 : 0, NC4 = (NC + 3) / 4 * 4;
+    return 3 * MMA_MP + 2 * MMA_MP + (size_t)(1 + np) * MMA_TG * MMA_MP + MMA_WAVES * MMA_MP + MMA_GP + MMA_MP +
+           2 * MMA_GP + (size_t)np * MMA_MP + (size_t)MMA_GP * np * NC + ((size_t)NC4 * MMA_MP * tsize + 7) / 8;
 }
 
 #ifndef CHAMP_MMA_WPE
-#define CHAMP_MMA_WPE 2
+#define CHAMP_MMA_WPE 3
 #endif
 // T: arithmetic type of the Jastrow terms and of the matrix cores (double on
-// the FP64 path, float on the mixed path); sums and the psi ratio are double.
+// the FP64 path, float on the mixed path); the sums over points, centres and
+// partners that the split takes out of the product are double.
 template <int NORDC, typename T>
 __global__ void __launch_bounds__(MMA_THREADS) CHAMP_WAVES_PER_EU(CHAMP_MMA_WPE) k_nonloc_mma(HArgs a)
 {
     HIP_DYNAMIC_SHARED(double, lds)
-    constexpr EenTable<NORDC> ET{};
+    constexpr int NP = een_nsep<NORDC>();
     static_assert(MMA_GP * 12 <= MMA_MP, "group size");
     const int tid = threadIdx.x, lane = tid % WAVE, wv = tid / WAVE;
-    const int NE = a.NE, NC = a.NC, NQ = a.NQ, NB = a.NB, NRI = a.NRI;
+    const int NE = a.NE, NC = a.NC, NQ = a.NQ, NC4 = (NC + 3) / 4 * 4;
     // the Jastrow parameters and the centres' types in LDS (read before use
     // behind the group loop's first barrier): every centre step of every item
     // reads a type's e-e-n coefficients, every epilogue entry the e-e ones
@@ -466,40 +527,21 @@ __global__ void __launch_bounds__(MMA_THREADS) CHAMP_WAVES_PER_EU(CHAMP_MMA_WPE)
     for (int t = tid; t < (int)(sizeof(JasParams) / 8); t += MMA_THREADS)
         reinterpret_cast<unsigned long long *>(&sJ)[t] = reinterpret_cast<const unsigned long long *>(a.jas)[t];
     for (int t = tid; t < NC; t += MMA_THREADS) sT[t] = a.iwctype[t];
+    __shared__ T sEE[2 * EE_NP];
+    ee_table<T>(*a.jas, sEE);
     const JasParams &jp = sJ;
     const double kapd = a.jas->kap;  // read directly: sJ is complete only after a barrier
-    const T kap = (T)kapd;
     double *XP = lds;                                          // [MP][3]
-    double *SP = XP + 3 * MMA_MP;                              // [3][MP]: e-e + e-n, e-e-n, psi ratio
-    double *TP = SP + 3 * MMA_MP;                              // [2][TG][MP] partial sums
-    double *SW = TP + 2 * MMA_TG * MMA_MP;                     // [WAVES][MP]
+    double *SP = XP + 3 * MMA_MP;                              // [2][MP]: e-n and point sums, e-e and e-e-n
+    double *TP = SP + 2 * MMA_MP;                              // [1 + NP][TG][MP] partial sums
+    double *SW = TP + (size_t)(1 + NP) * MMA_TG * MMA_MP;      // [WAVES][MP]
     double *FI = SW + MMA_WAVES * MMA_MP;                      // [GP]
     int *IPT = (int *)(FI + MMA_GP);                           // [MP] electron of each point
     int *PI = IPT + 2 * MMA_MP;                                // [GP][4]: i, ic
-    T *XQ = (T *)(PI + 8 * MMA_GP);                            // [NC][MP] switched point-centre distances
-    double *GR = (double *)PI + 4 * MMA_GP + ((size_t)NC * MMA_MP * sizeof(T) + 7) / 8;  // [MP][NC] point-centre r
-    int *GI = (int *)(GR + (size_t)NC * MMA_MP);               // [MP][NC] grid interval of r
-    double *PS = TP;                                           // [PS][MP] psi-ratio partials
-    // the radial instances in slot order (centre, type, radial function, AO range)
-    // and their AOs, staged once per block: the psi-ratio lanes read them per
-    // (point, instance), so from global memory their latency dominated that phase
-    int *SMI = GI + (size_t)NC * MMA_MP;                       // [NRI][8]
-    double *SRM = (double *)(SMI + (size_t)NRI * 8);           // [NRI] cut radius
-    int *SAO = (int *)(SRM + NRI);                             // [NB][2] slm code, AO index
-    const bool psi_ext = a.psi_ext != 0;  // psi ratios from k_nonloc_psi
-    if (!psi_ext) {
-        for (int sidx = tid; sidx < NRI; sidx += MMA_THREADS) {
-            const int ri = a.ri_perm[sidx];
-            SMI[8 * sidx] = a.ri_cent[ri]; SMI[8 * sidx + 1] = a.ri_type[ri]; SMI[8 * sidx + 2] = a.ri_rad[ri];
-            SMI[8 * sidx + 3] = a.ri_aoff[ri]; SMI[8 * sidx + 4] = a.ri_aoff[ri + 1];
-            SRM[sidx] = a.ri_rmax[ri];
-        }
-        for (int k = tid; k < NB; k += MMA_THREADS) {
-            const int m = a.ri_aol[k];
-            SAO[2 * k] = a.ao_slm[m];
-            SAO[2 * k + 1] = m;
-        }
-    }
+    double *XK = FI + MMA_GP + MMA_MP + 2 * MMA_GP;            // [NP][MP] X_k of each point
+    double *D0 = XK + NP * MMA_MP;                             // [GP][NP][NC] sum_j C_0n(y_jb) - C_0n(y_ib)
+    T *XQ = (T *)(D0 + (size_t)MMA_GP * NP * NC);              // [NC4][MP] switched point-centre distances
+    for (int t = NC * MMA_MP + tid; t < NC4 * MMA_MP; t += MMA_THREADS) XQ[t] = T(0);
 
     const int G = gridDim.x, bk = blockIdx.x;
     const int nx = (G % 8 == 0) ? 8 : 1, gx = G / nx, xcd = bk % nx, g0 = bk / nx;
@@ -525,12 +567,16 @@ __global__ void __launch_bounds__(MMA_THREADS) CHAMP_WAVES_PER_EU(CHAMP_MMA_WPE)
         }
         __syncthreads();
         for (int t = tid; t < MMA_MP; t += MMA_THREADS) IPT[t] = t < npts ? PI[4 * (t / NQ)] : -1;
-        for (int t = tid; t < 3 * npts; t += MMA_THREADS) {
+        for (int t = tid; t < 3 * MMA_MP; t += MMA_THREADS) {
             const int pt = t / 3, k = t % 3, p = pt / NQ, q = pt % NQ;
-            const int i = PI[4 * p], ic = PI[4 * p + 1];
-            const double ren = a.r_en[((size_t)w * NC + ic) * NE + i];
-            const double *qv = (k == 0 ? a.xq : (k == 1 ? a.yq : a.zq)) + (size_t)w * NQ;
-            XP[t] = ren * qv[q] + a.cent[3 * ic + k];
+            double v = 0.0;
+            if (pt < npts) {
+                const int i = PI[4 * p], ic = PI[4 * p + 1];
+                const double ren = a.r_en[((size_t)w * NC + ic) * NE + i];
+                const double *qv = (k == 0 ? a.xq : (k == 1 ? a.yq : a.zq)) + (size_t)w * NQ;
+                v = ren * qv[q] + a.cent[3 * ic + k];
+            }
+            XP[t] = v;
         }
         if (wv < np) {  // sum_j F[i][j] of each pair
             const double *F = a.fso + ((size_t)w * NE + PI[4 * wv]) * NE;
@@ -539,12 +585,25 @@ __global__ void __launch_bounds__(MMA_THREADS) CHAMP_WAVES_PER_EU(CHAMP_MMA_WPE)
             fs = wave_sum(fs);
             if (lane == 0) FI[wv] = fs;
         }
+        for (int t = tid; t < np * NC; t += MMA_THREADS) {  // the pairs' weights of x^n (k = 0)
+            const int p = t / NC, b = t % NC;
+            double yp[NORDC + 1];
+            een_powers<NORDC>(1.0 - kapd * a.rr_en[((size_t)w * NC + b) * NE + PI[4 * p]], yp);
+            const double *ct = jp.c[sT[b]];
+#pragma unroll
+            for (int n = 1; n <= NP; n++)
+                D0[((size_t)p * NP + n - 1) * NC + b] =
+                    a.een_t0[((size_t)w * NP + n - 1) * NC + b] - een_coupled<NORDC>(ct, yp, 0, n);
+        }
         __syncthreads();
 
-        // ---- points: x_qb and the e-n sums, the e-e sums
+        // ---- points: x_qb, the e-n sums and the parts of the e-e-n sum that
+        // hold one point-centre distance (X_k; the k = 0 terms)
         {
             const int pt = tid % MMA_MP, tg = tid / MMA_MP;
-            double sen = 0.0, see = 0.0;
+            double sen = 0.0, sx[NP];
+#pragma unroll
+            for (int k = 0; k < NP; k++) sx[k] = 0.0;
             if (tg < MMA_TG) {
                 const bool live = pt < npts;
                 const int p = live ? pt / NQ : 0;
@@ -557,63 +616,61 @@ __global__ void __launch_bounds__(MMA_THREADS) CHAMP_WAVES_PER_EU(CHAMP_MMA_WPE)
                         const T e0 = (T)(px - a.cent[3 * b]), e1 = (T)(py - a.cent[3 * b + 1]), e2 = (T)(pz - a.cent[3 * b + 2]);
                         T r2 = 0;
                         r2 = r2 + e0 * e0; r2 = r2 + e1 * e1; r2 = r2 + e2 * e2;
-                        const T rq = b == ic ? (T)a.r_en[((size_t)w * NC + ic) * NE + i] : sqrt(r2);
-                        const T rr = scale_r<T>(kap, rq);
-                        xq = switched_from<T>(kapd, rq, rr);
-                        sen += (double)en_term<T>(jp, a.iwctype[b], rr, xq);
+                        const T rq = b == ic ? (T)a.r_en[((size_t)w * NC + ic) * NE + i] : sqrt_inner(r2);
+                        xq = exp_neg((T)(-kapd * (double)rq));
+                        const T rr = (T(1) - xq) * (T)jp.asymp_r;
+                        sen += (double)en_term<T>(jp, sT[b], rr, xq);
+                        double xp[NORDC + 1];
+                        een_powers<NORDC>((double)xq, xp);
+                        een_uncoupled<NORDC>(jp.c[sT[b]], xp, sx);
+#pragma unroll
+                        for (int n = 1; n <= NP; n++) sen += xp[n] * D0[((size_t)p * NP + n - 1) * NC + b];
                     }
                     XQ[(size_t)b * MMA_MP + pt] = xq;
                 }
-                // with the e-e-n terms on the matrix cores (NORDC > 1) the e-e
-                // terms are added in their epilogue, which forms u_qj anyway
-                if (NORDC <= 1 && live)
-                    for (int j = tg; j < NE; j += MMA_TG) {
-                        if (j == i) continue;
-                        const T d0 = (T)(xw[j] - px), d1 = (T)(xw[NE + j] - py), d2 = (T)(xw[2 * NE + j] - pz);
-                        T r2 = 0;
-                        r2 = r2 + d0 * d0; r2 = r2 + d1 * d1; r2 = r2 + d2 * d2;
-                        const T rjq = sqrt(r2);
-                        const T u = scale_r<T>(kap, rjq);
-                        see += (double)ee_term<T>(jp, a.NUP, i, j, u, switched_from<T>(kapd, rjq, u));
-                    }
-                TP[tg * MMA_MP + pt] = see;
-                TP[(MMA_TG + tg) * MMA_MP + pt] = sen;
+                TP[tg * MMA_MP + pt] = sen;
+#pragma unroll
+                for (int k = 0; k < NP; k++) TP[((k + 1) * MMA_TG + tg) * MMA_MP + pt] = sx[k];
             }
         }
         __syncthreads();
-        for (int pt = tid; pt < MMA_MP; pt += MMA_THREADS) {
+        for (int t = tid; t < (1 + NP) * MMA_MP; t += MMA_THREADS) {
+            const int k = t / MMA_MP, pt = t % MMA_MP;
             double v = 0.0;
-            for (int tg = 0; tg < MMA_TG; tg++) v += TP[tg * MMA_MP + pt];
-            for (int tg = 0; tg < MMA_TG; tg++) v += TP[(MMA_TG + tg) * MMA_MP + pt];
-            SP[pt] = v;
+            for (int tg = 0; tg < MMA_TG; tg++) v += TP[(k * MMA_TG + tg) * MMA_MP + pt];
+            if (k == 0) SP[pt] = v;
+            else XK[(k - 1) * MMA_MP + pt] = v;
         }
+        __syncthreads();
 
-        // ---- e-e-n on the matrix cores: items (16 partners, all row tiles) over
-        // the waves; each wave sums its items into its own row of SW
+        // ---- e-e and e-e-n: items (16 partners x 16 points) in contiguous runs of
+        // equal length per wave; the wave's sums go to its own row of SW
         {
-            double *swv = SW + wv * MMA_MP;
-            for (int pt = lane; pt < MMA_MP; pt += WAVE) swv[pt] = 0.0;
-            __syncwarp();
-            if constexpr (NORDC > 1) {
-                // half-tiles (16 partners x half the centres) dealt in contiguous
-                // runs of equal length to the waves; two halves of one tile in a
-                // run make one item over all centres
-                const int NT = (NE + 15) / 16, nh = 2 * NT, per = (nh + MMA_WAVES - 1) / MMA_WAVES;
-                const int ncm = min(NC, ((NC / 2 + 3) / 4) * 4);  // centres of the first half (a multiple of 4)
-                const int h_hi = min(nh, (wv + 1) * per);
-                for (int h = wv * per; h < h_hi;) {
-                    const int tile = h / 2;
-                    if (h % 2 == 0 && h + 1 < h_hi) {
-                        mma_item<NORDC, T>(a, w, tile * 16, 0, NC, npts, XP, XQ, IPT, swv, true, sJ, sT);
-                        h += 2;
-                    } else {
-                        mma_item<NORDC, T>(a, w, tile * 16, h % 2 ? ncm : 0, h % 2 ? NC : ncm, npts, XP, XQ, IPT, swv,
-                                           h % 2 == 0, sJ, sT);
-                        h += 1;
-                    }
-                    __syncwarp();
-                }
+            double psum[MMA_MT][4];
+#pragma unroll
+            for (int mt = 0; mt < MMA_MT; mt++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) psum[mt][r] = 0.0;
+            const int NT = (NE + 15) / 16, RT = (npts + 15) / 16, items = NT * RT;
+            const int per = (items + MMA_WAVES - 1) / MMA_WAVES, it_hi = min(items, (wv + 1) * per);
+            for (int it = wv * per; it < it_hi;) {
+                const int tile = it / RT, m0 = it - tile * RT, cnt = min(RT - m0, it_hi - it);
+                if (cnt == 3)
+                    mma_item<NORDC, T, 3>(a, w, tile * 16, 0, npts, XP, XQ, XK, IPT, psum, jp, sT, sEE);
+                else if (cnt == 2)
+                    mma_item<NORDC, T, 2>(a, w, tile * 16, m0, npts, XP, XQ, XK, IPT, psum, jp, sT, sEE);
+                else
+                    mma_item<NORDC, T, 1>(a, w, tile * 16, m0, npts, XP, XQ, XK, IPT, psum, jp, sT, sEE);
+                it += cnt;
             }
+            // over the 16 partners of a tile (lanes of equal l / 16)
+#pragma unroll
+            for (int mt = 0; mt < MMA_MT; mt++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const double v = row16_sum(psum[mt][r]);
+                    if (lane % 16 == 0) SW[wv * MMA_MP + mt * 16 + Mma<T>::row(r, lane / 16)] = v;
+                }
         }
         __syncthreads();
         for (int pt = tid; pt < MMA_MP; pt += MMA_THREADS) {
@@ -621,57 +678,6 @@ __global__ void __launch_bounds__(MMA_THREADS) CHAMP_WAVES_PER_EU(CHAMP_MMA_WPE)
             for (int k = 0; k < MMA_WAVES; k++) v += SW[k * MMA_MP + pt];
             SP[MMA_MP + pt] = v;
         }
-
-        // ---- psi ratio of every point: sum_m phi_m(x_q) W[i][m].  The point-centre
-        // distances and grid intervals first, then lanes over (point, radial
-        // instance): a lane forms the instance's radial value at its point and
-        // dots the instance's angular factors with the W row.  Instances are
-        // taken in order of their AO count (ri_perm), so the lanes of a wave
-        // mostly run the same number of AOs.
-        __syncthreads();  // SW and the point-phase partials are free
-        if (!psi_ext) {
-        for (int t = tid; t < npts * NC; t += MMA_THREADS) {
-            const int q = t / NC, c = t % NC, p = q / NQ;
-            const double *xp = XP + 3 * q;
-            const double e0 = xp[0] - a.cent[3 * c], e1 = xp[1] - a.cent[3 * c + 1], e2 = xp[2] - a.cent[3 * c + 2];
-            double r2 = 0;
-            r2 = r2 + e0 * e0; r2 = r2 + e1 * e1; r2 = r2 + e2 * e2;
-            const double rqd = c == PI[4 * p + 1] ? a.r_en[((size_t)w * NC + c) * NE + PI[4 * p]] : sqrt(r2);
-            GR[t] = rqd;
-            GI[t] = grid_jx(a.tab, rqd);
-        }
-        __syncthreads();
-        {
-            const int q = tid % MMA_MP, slot = tid / MMA_MP;
-            double part = 0.0;
-            if (slot < MMA_PS && q < npts) {
-                const double px = XP[3 * q], py = XP[3 * q + 1], pz = XP[3 * q + 2];
-                const double *Wm = a.wmat + ((size_t)w * NE + IPT[q]) * NB;
-                const double *gr = GR + (size_t)q * NC;
-                const int *gi = GI + (size_t)q * NC;
-                for (int sidx = slot; sidx < NRI; sidx += MMA_PS) {
-                    const int *mi = SMI + 8 * sidx;
-                    const int cen = mi[0];
-                    const double r = gr[cen];
-                    if (!(r <= SRM[sidx])) continue;  // beyond the shell's cut radius: its AOs are exactly zero
-                    double wfv[3] = {0.0, 0.0, 0.0};
-                    splfit_jx<double>(a.tab, mi[1], mi[2], r, gi[cen], wfv, 0);
-                    const double d0 = px - a.cent[3 * cen], d1 = py - a.cent[3 * cen + 1], d2 = pz - a.cent[3 * cen + 2];
-                    double sa = 0.0;
-                    for (int k = mi[3]; k < mi[4]; k++)
-                        sa += slm_value<double>(slm_decode(SAO[2 * k]), d0, d1, d2) * Wm[SAO[2 * k + 1]];
-                    part += sa * wfv[0];
-                }
-            }
-            PS[tid] = part;
-        }
-        __syncthreads();
-        for (int q = tid; q < npts; q += MMA_THREADS) {
-            double v = 0.0;
-            for (int k = 0; k < MMA_PS; k++) v += PS[k * MMA_MP + q];
-            SP[2 * MMA_MP + q] = v;
-        }
-        }  // !psi_ext
         __syncthreads();
 
         // ---- the vpsp_det terms (nonloc.f90:248-274): a thread per point
@@ -692,7 +698,7 @@ __global__ void __launch_bounds__(MMA_THREADS) CHAMP_WAVES_PER_EU(CHAMP_MMA_WPE)
             for (int l = 1; l <= lp - 1; l++)
                 term_radial = term_radial + yl0(l, costh) * a.pair_vps[slot * CHAMP_MPS_L + l - 1];
             const double trj = term_radial * a.ecp->wq[q] * exp(fsumn);
-            TRJ[pt] = trj * (psi_ext ? a.pair_psi[slot * NQ + q] : SP[2 * MMA_MP + pt]);
+            TRJ[pt] = trj * a.pair_psi[slot * NQ + q];
             // t_vpsp of the point (nonloc.f90:297) for DMC's T-moves
             if (a.tstore) a.pair_psi[slot * NQ + q] = TRJ[pt];
         }
@@ -709,11 +715,12 @@ __global__ void __launch_bounds__(MMA_THREADS) CHAMP_WAVES_PER_EU(CHAMP_MMA_WPE)
 // ------------------------------------------------------------------------
 // The psi ratio of every quadrature point on its own: sum_m phi_m(x_q) W[i][m]
 // (the orbital part of nonloc.f90:224-247, contracted with the inverse row
-// once per electron: wmat).  The same groups of MMA_GP pairs and the same lane
-// form as the psi phase of k_nonloc_mma, in a kernel of few registers and
-// small LDS, so that more waves hide its table and W loads.  Results go to
-// pair_psi[slot][q] for k_nonloc_mma (psi_ext).
+// once per electron: wmat), for the groups of MMA_GP pairs of k_nonloc_mma:
+// lanes over (point, radial-instance slot).  A kernel of few registers and
+// small LDS of its own, so that more waves hide its table and W loads.
+// Results go to pair_psi[slot][q] for k_nonloc_mma.
 constexpr int PSI_MP = MMA_MP, PSI_THREADS = MMA_THREADS;
+constexpr int MMA_PS = PSI_THREADS / PSI_MP;
 
 __host__ __device__ __forceinline__ size_t psi_lds_bytes(int NC, int NB, int NRI)
 {
@@ -825,10 +832,6 @@ __global__ void __launch_bounds__(PSI_THREADS) k_nonloc_psi(HArgs a)
     }
 }
 
-#ifndef CHAMP_NL_SPLIT
-#define CHAMP_NL_SPLIT 1
-#endif
-
 static int launch_psi(champ_ctx *c, const HArgs &a)
 {
     const size_t lds = psi_lds_bytes(c->NC, c->NB, c->NRI);
@@ -845,25 +848,14 @@ static int launch_psi(champ_ctx *c, const HArgs &a)
 }
 
 template <int NORDC, typename T>
-static int launch_mma(champ_ctx *c, const HArgs &a0)
+static int launch_mma(champ_ctx *c, const HArgs &a)
 {
-    HArgs a = a0;
-    const bool split = CHAMP_NL_SPLIT && psi_lds_bytes(c->NC, c->NB, c->NRI) <= 160 * 1024;
     int slot;
-    if (split) {
-        tbegin(c, K_HPSI_PSI, &slot);
-        const int rc = launch_psi(c, a);
-        tend(c, slot);
-        if (rc) return rc;
-        a.psi_ext = 1;
-    }
-    // without the psi phase the tables after XQ (point-centre distances,
-    // instances, AOs) are not used
-    const size_t lds = (mma_lds_doubles(c->NC, c->NB, c->NRI, (int)sizeof(T)) -
-                        (split ? (size_t)c->NC * MMA_MP + ((size_t)c->NC * MMA_MP * 4 + 7) / 8 + (size_t)c->NRI * 4 +
-                                     (size_t)c->NRI + (size_t)c->NB
-                               : 0)) *
-                       sizeof(double);
+    tbegin(c, K_HPSI_PSI, &slot);
+    const int rc = launch_psi(c, a);
+    tend(c, slot);
+    if (rc) return rc;
+    const size_t lds = mma_lds_doubles(c->NC, NORDC, (int)sizeof(T)) * sizeof(double);
     if (lds > 160 * 1024) {
         set_error("nonloc: the quadrature kernel's LDS tables exceed 160 KB for this system");
         return CHAMP_ERR_UNSUPPORTED;
@@ -927,13 +919,20 @@ static int launch_t(champ_ctx *c, const HArgs &a)
 #define CHAMP_NL_MMA 1
 #endif
 
+// the matrix-core form: up to 12 points per pair (48 points per group), an
+// e-e-n polynomial, and the LDS of both its kernels within 160 KB beside the
+// static arrays (JasParams and 128 types, nuclear positions)
+bool nonloc_on_matrix_cores(const champ_ctx *c)
+{
+    const size_t most = 160 * 1024 - sizeof(JasParams) - 3 * 128 * sizeof(double) - 512;
+    return CHAMP_NL_MMA && c->tune_nonloc != 1 && c->NQ <= 12 && c->hjas.nordc >= 2 && c->hjas.nordc <= 5 &&
+           mma_lds_doubles(c->NC, c->hjas.nordc, c->prec == CHAMP_PREC_MIXED ? 4 : 8) * 8 <= most &&
+           psi_lds_bytes(c->NC, c->NB, c->NRI) <= most;
+}
+
 int launch_nonloc(champ_ctx *c, const HArgs &a)
 {
-    // the matrix-core form: up to 12 points per pair (48 points per group) and
-    // its LDS within 160 KB
-    const bool mixed = c->prec == CHAMP_PREC_MIXED;
-    const bool mma = CHAMP_NL_MMA && c->tune_nonloc != 1 && c->NQ <= 12 && c->hjas.nordc >= 2 && c->hjas.nordc <= 5 &&
-                     mma_lds_doubles(c->NC, c->NB, c->NRI, mixed ? 4 : 8) * 8 <= 160 * 1024;
+    const bool mixed = c->prec == CHAMP_PREC_MIXED, mma = nonloc_on_matrix_cores(c);
     if (mma && mixed) {
         switch (c->hjas.nordc) {
         case 2: return launch_mma<2, float>(c, a);

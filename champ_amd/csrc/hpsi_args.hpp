@@ -23,10 +23,11 @@ struct HArgs {
     int *pair_count, *pair_off, *pair_total, *pair_e, *pair_c, *nxquad;
     int *grp_off;  // [W+1] groups of NL_GROUP pairs per walker (prefix sums); pair_total[1] = groups
     double *pair_vps, *pair_val;
-    double *pair_psi;  // [W*cap][NQ] psi ratios from k_nonloc_psi (psi_ext), else unused
+    double *pair_psi;  // [W*cap][NQ] psi ratios from k_nonloc_psi, read by k_nonloc_mma
     float2 *enp;       // mixed path: the FP32 partner pair table, else null
+    double *een_ys, *een_t0;  // [W][nordc-1][NE], [W][nordc-1][NC] split e-e-n sums (een_poly.hpp) of the quadrature
+    int rrt;           // write rrT (the vector-pipe quadrature form reads it)
     int tstore;        // keep each point's t_vpsp (its term of the ECP sum) in pair_psi
-    int psi_ext;
     double *rrT;  // [W][NE][NC] scaled e-n distances, centre index innermost
     int NRI;      // radial instances (centre, radial function)
     const int *ri_cent, *ri_type, *ri_rad, *ao_ri;
@@ -56,7 +57,8 @@ inline HArgs hargs(champ_ctx *c)
     a.pe_local = c->pe_local; a.vpsp = c->vpsp; a.aoall = c->aoall; a.orball = c->orball; a.wmat = c->wmat;
     a.pair_count = c->pair_count; a.pair_off = c->pair_off; a.pair_total = c->pair_total; a.pair_e = c->pair_e;
     a.pair_c = c->pair_c; a.nxquad = c->nxquad; a.grp_off = c->grp_off; a.pair_vps = c->pair_vps; a.pair_val = c->pair_val;
-    a.pair_psi = c->pair_psi; a.psi_ext = 0;
+    a.pair_psi = c->pair_psi;
+    a.een_ys = c->een_ys; a.een_t0 = c->een_t0; a.rrt = 1;
     a.enp = c->enp;
     a.tstore = c->tstore;
     a.rrT = c->rrT;
@@ -101,6 +103,7 @@ constexpr size_t SLATER_STATIC_LDS = 512 * sizeof(int) + 512 * sizeof(double) + 
 
 // ECP quadrature over the active (electron, centre) pairs (engine_nonloc.hip)
 int launch_nonloc(champ_ctx *c, const HArgs &a);
+bool nonloc_on_matrix_cores(const champ_ctx *c);  // the form launch_nonloc takes
 constexpr int NL_GROUP = 4;  // pairs of one walker per block of the matrix-core quadrature kernel
 
 }  // namespace champ

@@ -113,6 +113,24 @@ inline int __builtin_amdgcn_readfirstlane(int v)
         }
     return (int)(uint32_t)all[base];
 }
+// hardware estimates of 1 / sqrt(x) and 1 / x: about 27 good bits
+inline double __builtin_amdgcn_rsq(double x) { return (1.0 / std::sqrt(x)) * (1.0 + 0x1p-27); }
+inline double __builtin_amdgcn_rcp(double x) { return (1.0 / x) * (1.0 + 0x1p-27); }
+inline void __builtin_amdgcn_sched_barrier(int) {}  // scheduling only
+// Register move between the lanes of a row of 16 by its DPP control word:
+// quad_perm (0x00-0xff), row_mirror (0x140) and row_half_mirror (0x141)
+inline int __builtin_amdgcn_mov_dpp(int v, int ctrl, int, int, bool)
+{
+    uint64_t all[64];
+    emu::wave_exchange((uint64_t)(uint32_t)v, all);
+    const int l = emu::tctx.lane % 64;
+    int src = l;
+    if (ctrl < 0x100) src = (l & ~3) | ((ctrl >> (2 * (l & 3))) & 3);
+    else if (ctrl == 0x140) src = (l & ~15) | (15 - (l & 15));
+    else if (ctrl == 0x141) src = (l & ~7) | (7 - (l & 7));
+    else { fprintf(stderr, "emu: DPP control %x not modelled\n", ctrl); abort(); }
+    return (int)(uint32_t)all[src];
+}
 // FP64 MFMA 16x16x4: lane l supplies A[l % 16][l / 16] and B[l / 16][l % 16]
 // and holds D[4 r + l / 16][l % 16] in accumulator element r = 0..3 (the
 // layout measured on gfx950 with a one-hot probe of A and B)

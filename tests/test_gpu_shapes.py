@@ -1,0 +1,47 @@
+"""Engine against the oracle on molecules whose sizes cut the kernels' tiles: electron
+counts around 16 and 64, centre counts that 4 does not divide, few quadrature pairs,
+unequal spins, and e-e-n orders 2, 3 and 5."""
+import numpy as np
+import pytest
+
+from champ_amd import system as S
+from champ_amd.engine import PREC_FP64, PREC_MIXED, Engine
+from oracle import ffi
+from tests.gpu_helpers import ENGINE_LIB, relnorm
+
+pytestmark = pytest.mark.gpu
+
+# heavy atoms, hydrogens, electrons, e-e-n order, pseudopotential
+SHAPES = [(2, 0, 2, 4, True), (2, 1, 9, 2, True), (3, 2, 17, 3, True), (5, 0, 33, 5, True), (4, 3, 16, 4, True),
+          (9, 4, 65, 4, True), (3, 3, 15, 5, False)]
+
+
+def molecule(nheavy, nh, nelec, order, ecp):
+    return S.make_system("shape", nheavy, nh, nelec, "ssppd", "sp", nloc=4 if ecp else 0, nordc=order)
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "-".join(map(str, s)))
+@pytest.mark.parametrize("prec", [PREC_FP64, PREC_MIXED])
+def test_hpsi_of_odd_shapes(require_gpu, shape, prec):
+    sy = molecule(*shape)
+    nw = 3
+    x = sy.initial_walkers(nw, seed=4)
+    eng = Engine(sy, nw, precision=prec, lib_path=ENGINE_LIB)
+    eng.set_walkers(x)
+    g = eng.hpsi()
+    # FP64: the rounding of sums of a few thousand terms, and of a Slater inverse
+    # of condition up to 1e6 in the energies; mixed: FP32 terms summed in FP64
+    tol_j, tol_e = (1e-12, 1e-9) if prec == PREC_FP64 else (2e-6, 2e-5)
+    ref = []
+    for w in range(nw):
+        o = ffi.walker(sy)
+        o.set_x(x[w])
+        if sy.nloc:
+            o.set_quad(sy.xq0, sy.yq0, sy.zq0)
+        ref.append(o.hpsi())
+        assert relnorm(eng.array("vj")[w], o.vj()) < max(tol_j, 1e-12) * 10
+    for key, tol in (("psij", tol_j), ("ekin", tol_e), ("energy", tol_e)):
+        r = np.array([d[key] for d in ref])
+        # the terms of E_L cancel: relative to their own size
+        scale = np.maximum(1.0, np.abs(r)) if key != "energy" else np.maximum(np.abs(r), np.abs([d["ekin"] for d in ref]))
+        assert np.all(np.abs(g[key] - r) <= tol * np.maximum(1.0, scale)), (key, g[key], r)
