@@ -359,6 +359,19 @@ __device__ __forceinline__ void ao_eval(const SplineTab &tab, int it, int irad, 
     ao_combine<T>(l, rx, ry, rz, r, wfv, ider, out);
 }
 
+// Weights of a radius in its grid interval jx (1 <= jx < nr): the spline value
+// is aa y0 + bb y1 + cc s0 + dd s1 (splfit_jx with the interval's factors formed
+// once for all shells of a centre).
+__device__ __forceinline__ void spline_weights(const SplineTab &tab, double r, int jx, double w[4])
+{
+    const double ref0 = tab.gref[2 * jx], ref1 = tab.gref[2 * jx + 1];
+    const double delh = ref1 - ref0, delhi = div_inner(1.0, delh), h6 = delh * delh * (1.0 / 6.0);
+    w[0] = (ref1 - r) * delhi;
+    w[1] = (r - ref0) * delhi;
+    w[2] = w[0] * (w[0] * w[0] - 1.0) * h6;
+    w[3] = w[1] * (w[1] * w[1] - 1.0) * h6;
+}
+
 // ----------------------------------------------------------------- Jastrow
 #define CHAMP_MAXCT 4
 #define CHAMP_MAXT 32

@@ -280,17 +280,64 @@ extern "C" int champ_gpu_init(champ_ctx **ctxp, const champ_system_t *s, int32_t
         TRY(upload(&c->ri_cent, ric.data(), ric.size())); TRY(upload(&c->ri_type, rit.data(), rit.size()));
         TRY(upload(&c->ri_rad, rir.data(), rir.size())); TRY(upload(&c->ri_rmax, rirm.data(), rirm.size()));
         TRY(upload(&c->ao_ri, aori.data(), NB));
-        // each instance's AOs, and the instances in decreasing order of their AO count
-        std::vector<int> aoff(c->NRI + 1, 0), aol(NB), perm(c->NRI);
-        for (int m = 0; m < NB; m++) aoff[aori[m] + 1]++;
-        for (int r = 0; r < c->NRI; r++) aoff[r + 1] += aoff[r];
-        std::vector<int> fill(aoff.begin(), aoff.end() - 1);
-        for (int m = 0; m < NB; m++) aol[fill[aori[m]]++] = m;
-        for (int r = 0; r < c->NRI; r++) perm[r] = r;
-        std::stable_sort(perm.begin(), perm.end(),
-                         [&](int x, int y) { return aoff[x + 1] - aoff[x] > aoff[y + 1] - aoff[y]; });
-        TRY(upload(&c->ri_perm, perm.data(), c->NRI)); TRY(upload(&c->ri_aoff, aoff.data(), c->NRI + 1));
-        TRY(upload(&c->ri_aol, aol.data(), NB));
+    }
+    // the same by centre type (ShellTab): spline tables node by node, AO segments
+    {
+        const int nrb = s->nrbas_max, nr = s->nr;
+        std::vector<double> tab((size_t)NCT * nr * nrb * 2, 0.0), trm(NCT, 0.0);
+        std::vector<int> soff(NCT + 1, 0), seg, sao, tco(NCT + 1, 0), tcc, first(NC, 0);
+        const int lo[4] = {1, 2, 5, 11}, n[4] = {1, 3, 6, 10};
+        for (int it = 0; it < NCT; it++) {
+            for (int ir = 0; ir < s->nrbas[it]; ir++) {
+                const size_t row = ((size_t)it * nrb + ir) * nr;
+                for (int j = 0; j < nr; j++) {
+                    double *t = &tab[(((size_t)it * nr + j) * nrb + ir) * 2];
+                    t[0] = s->rwf[row + j];
+                    t[1] = s->d2rwf[row + j];
+                }
+                std::vector<int> left;  // the shell's AOs, type-local
+                for (int i = 0; i < s->nbastyp[it]; i++)
+                    if (s->iwrwf[it * s->nbastyp_max + i] == ir) left.push_back(i);
+                if (!left.empty()) trm[it] = std::max(trm[it], s->rmaxwf[it * nrb + ir]);
+                for (int kind = 0; kind < 4; kind++) {  // whole sets, as often as they occur
+                    for (;;) {
+                        std::vector<int> set;
+                        for (int k = 0; k < n[kind]; k++)
+                            for (int i : left)
+                                if (s->iwlbas[it * s->nbastyp_max + i] == lo[kind] + k) { set.push_back(i); break; }
+                        if ((int)set.size() < n[kind]) break;
+                        seg.insert(seg.end(), {ir, kind, (int)sao.size(), 0});
+                        sao.insert(sao.end(), set.begin(), set.end());
+                        for (int i : set) left.erase(std::find(left.begin(), left.end(), i));
+                    }
+                }
+                for (int i : left) {
+                    seg.insert(seg.end(), {ir, 4, (int)sao.size(), s->iwlbas[it * s->nbastyp_max + i]});
+                    sao.push_back(i);
+                }
+            }
+            soff[it + 1] = (int)seg.size() / 4;
+            for (int ic = 0; ic < NC; ic++)
+                if (s->iwctype[ic] == it) tcc.push_back(ic);
+            tco[it + 1] = (int)tcc.size();
+        }
+        for (int ic = 1; ic < NC; ic++) first[ic] = first[ic - 1] + s->nbastyp[s->iwctype[ic - 1]];
+        ShellTab &h = c->shl;
+        h.nct = NCT; h.nseg = (int)seg.size() / 4; h.nao = (int)sao.size();
+        // one allocation each for the doubles and the integers
+        const size_t ntab2 = tab.size();
+        tab.insert(tab.end(), trm.begin(), trm.end());
+        double *dt = nullptr;
+        TRY(upload(&dt, tab.data(), tab.size()));
+        h.tab = dt; h.rmax = dt + ntab2;
+        std::vector<int> pack;
+        size_t at[6];
+        const std::vector<int> *parts[6] = {&soff, &seg, &sao, &tco, &tcc, &first};
+        for (int k = 0; k < 6; k++) { at[k] = pack.size(); pack.insert(pack.end(), parts[k]->begin(), parts[k]->end()); }
+        int *di = nullptr;
+        TRY(upload(&di, pack.data(), pack.size()));
+        h.seg_off = di + at[0]; h.seg = di + at[1]; h.seg_ao = di + at[2]; h.tc_off = di + at[3];
+        h.tc_cent = di + at[4]; h.ao_first = di + at[5];
     }
     TRY(upload(&c->coef, s->coef, (size_t)NO * NB));
     if (precision == CHAMP_PREC_MIXED) {
@@ -393,7 +440,8 @@ extern "C" int champ_gpu_init(champ_ctx **ctxp, const champ_system_t *s, int32_t
         TRY(dalloc(&c->pair_psi, (size_t)W * c->pair_cap * std::max(c->NQ, 1)));
         TRY(dalloc(&c->rrT, (size_t)W * NE * NC));
         const size_t nsep = std::max(1, s->nordc - 1);
-        TRY(dalloc(&c->een_ys, (size_t)W * nsep * NE)); TRY(dalloc(&c->een_t0, (size_t)W * nsep * NC));
+        TRY(dalloc(&c->een_ys, (size_t)W * nsep * (NE + NC)));
+        c->een_t0 = c->een_ys + (size_t)W * nsep * NE;
     }
     TRY(dalloc(&c->pair_count, W)); TRY(dalloc(&c->pair_off, (size_t)W + 1)); TRY(dalloc(&c->pair_total, 2));
     TRY(dalloc(&c->grp_off, (size_t)W + 1));
@@ -443,8 +491,8 @@ extern "C" int champ_gpu_free(champ_ctx *c)
                     c->vjnT, c->fsumn, c->aomove, c->orbn, c->ratio, c->psidn, c->psijn, c->vnew, c->vold, c->acc,
                     c->esum_dev, c->aoall, c->orball, c->wmat, c->pair_count, c->pair_off, c->pair_total, c->grp_off,
                     c->pair_e, c->pair_c, c->pair_vps, c->pair_val, c->pair_psi, c->rrT, c->nxquad, c->ri_cent, c->ri_type,
-                    c->ri_rad, c->ri_rmax, c->ao_ri, c->gref, c->lu_ws, c->m6rec, c->ri_perm,
-                    c->ri_aoff, c->ri_aol, c->enp, c->gemm_tmp, c->een_ys, c->een_t0};
+                    c->ri_rad, c->ri_rmax, c->ao_ri, c->gref, c->lu_ws, c->m6rec, c->enp,
+                    (void *)c->shl.tab, (void *)c->shl.seg_off, c->gemm_tmp, c->een_ys};
     for (void *p : ptrs) if (p) hipFree(p);
     md_free(c);
     dmc_free(c);

@@ -11,6 +11,23 @@
 
 namespace champ {
 
+// The radial functions and AOs of each centre type, laid out for one lane per
+// (point, centre): a node's values of all shells lie together, so that the
+// lane's table reads fall into two or three lines, and the AOs of a shell form
+// segments of whole s, p, d or f sets (kind 0..3) or single monomials (kind 4,
+// with the slm code), the same for all lanes of a type.
+struct ShellTab {
+    const double *tab;       // [nctype][nr][nrbas_max][2] spline value and second derivative (owns rmax too)
+    const double *rmax;      // [nctype] largest cut radius of the type's shells
+    const int *seg_off;      // [nctype + 1] (owns the integer tables below)
+    const int *seg;          // [nseg][4] radial function, kind, first entry of seg_ao, slm code
+    const int *seg_ao;       // AO of the centre (type-local) per component, in slm's order
+    const int *tc_off;       // [nctype + 1] centres grouped by type
+    const int *tc_cent;      // [ncent]
+    const int *ao_first;     // [ncent] first AO of each centre
+    int nct, nseg, nao;      // types, segments and entries of seg_ao
+};
+
 struct DmcState;  // host side of a DMC population (engine_dmc.hip)
 
 struct EcpParams {
@@ -56,10 +73,10 @@ struct champ_ctx {
     int *ri_cent = nullptr, *ri_type = nullptr, *ri_rad = nullptr;  // [NRI]
     double *ri_rmax = nullptr;                                      // [NRI]
     int *ao_ri = nullptr;                                           // [NB] radial instance of each AO
-    int *ri_perm = nullptr;   // [NRI] instances in decreasing order of their AO count
-    int *ri_aoff = nullptr;   // [NRI+1] offsets of each instance's AOs in ri_aol
-    int *ri_aol = nullptr;    // [NB] AOs grouped by radial instance
     double *gref = nullptr;                                         // [nr][2] grid node radii
+    // the AOs of a centre by type, for the kernels that take a (point, centre)
+    // per lane (champ_gpu_init fills them)
+    champ::ShellTab shl{};
     int lu_every = 0;  // moves between FP64 recomputes of the Slater inverse inside a sweep (0: only in hpsi)
     int *ao_cent = nullptr, *ao_type = nullptr, *ao_rad = nullptr, *ao_slm = nullptr;  // [NB]
     double *coef = nullptr;          // [NO][NB]

@@ -95,6 +95,14 @@ template <typename T>
 inline T __shfl(T v, int src, int width = 64) { return emu::shfl_generic(v, src, width); }
 template <typename T>
 inline T __shfl_xor(T v, int mask, int width = 64) { return emu::shfl_generic(v, (emu::tctx.lane % width) ^ mask, width); }
+inline uint64_t __ballot(int p)
+{
+    uint64_t all[64], m = 0;
+    emu::wave_exchange(p ? 1 : 0, all);
+    for (int l = 0; l < 64; l++) m |= (all[l] & 1) << l;
+    return m;
+}
+inline int __popcll(uint64_t v) { return __builtin_popcountll(v); }
 // HIP's global integer min/max
 inline int min(int a, int b) { return a < b ? a : b; }
 inline int max(int a, int b) { return a > b ? a : b; }

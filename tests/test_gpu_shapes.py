@@ -45,3 +45,37 @@ def test_hpsi_of_odd_shapes(require_gpu, shape, prec):
         # the terms of E_L cancel: relative to their own size
         scale = np.maximum(1.0, np.abs(r)) if key != "energy" else np.maximum(np.abs(r), np.abs([d["ekin"] for d in ref]))
         assert np.all(np.abs(g[key] - r) <= tol * np.maximum(1.0, scale)), (key, g[key], r)
+
+
+def drop_ao(sy, it, i):
+    """The system without AO i of type it: its shell is no whole set any more."""
+    first = np.concatenate([[0], np.cumsum([sy.nbastyp[t] for t in sy.iwctype])])
+    gone = [first[c] + i for c, t in enumerate(sy.iwctype) if t == it]
+    sy.coef = np.ascontiguousarray(np.delete(sy.coef, gone, axis=1))
+    for name in ("iwrwf", "iwlbas"):
+        a = getattr(sy, name).copy()
+        a[it, i:-1] = a[it, i + 1:]
+        setattr(sy, name, a)
+    sy.nbastyp = sy.nbastyp.copy()
+    sy.nbastyp[it] -= 1
+    return sy
+
+
+@pytest.mark.parametrize("heavy,hyd,drop", [("spf", "s", None), ("sspd", "sp", (0, 3)), ("fd", "p", (0, 12)), ("s", "f", (1, 0))])
+def test_quadrature_of_shell_sets(require_gpu, heavy, hyd, drop):
+    """s, p, d and f sets, and shells that miss one of their monomials, in the
+    quadrature's psi ratio (all of E_L against the oracle)."""
+    sy = S.make_system("shells", 3, 2, 11, heavy, hyd, nloc=4, nordc=4)
+    if drop is not None:
+        sy = drop_ao(sy, *drop)
+    nw = 2
+    x = sy.initial_walkers(nw, seed=9)
+    eng = Engine(sy, nw, lib_path=ENGINE_LIB)
+    eng.set_walkers(x)
+    g = eng.hpsi()
+    for w in range(nw):
+        o = ffi.walker(sy)
+        o.set_x(x[w])
+        o.set_quad(sy.xq0, sy.yq0, sy.zq0)
+        d = o.hpsi()
+        assert abs(g["energy"][w] - d["energy"]) <= 1e-9 * max(1.0, abs(d["energy"]), abs(d["ekin"]))
