@@ -16,8 +16,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "libchamp_gpu.so")
 OBJDIR = os.path.join(HERE, "_build")
-SOURCES = ["engine_api.hip", "engine_kernels.hip", "engine_hpsi.hip", "engine_gemm.hip", "engine_nonloc.hip",
-           "engine_multidet.hip", "engine_dmc.hip", "engine_deriv.hip"]
+SOURCES = ["engine_api.hip", "engine_kernels.hip", "engine_sweep.hip", "engine_hpsi.hip", "engine_gemm.hip",
+           "engine_nonloc.hip", "engine_multidet.hip", "engine_dmc.hip", "engine_deriv.hip"]
 ARCH = os.environ.get("CHAMP_OFFLOAD_ARCH", "gfx950")
 
 HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
@@ -27,11 +27,13 @@ FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-result",
 ]
+# flags of single sources, with their reason in the source
+SOURCE_FLAGS = {"engine_sweep.hip": ["-mllvm", "-disable-machine-licm"]}
 
 
 def _compile(src: str, objdir: str = OBJDIR, defines: tuple = ()) -> str:
     obj = os.path.join(objdir, src.replace(".hip", ".o"))
-    cmd = [HIPCC, *FLAGS, *[f"-D{d}" for d in defines], "-c", os.path.join(CSRC, src), "-o", obj]
+    cmd = [HIPCC, *FLAGS, *SOURCE_FLAGS.get(src, []), *[f"-D{d}" for d in defines], "-c", os.path.join(CSRC, src), "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"hipcc failed for {src}:\n{r.stderr[-6000:]}")
@@ -40,7 +42,7 @@ def _compile(src: str, objdir: str = OBJDIR, defines: tuple = ()) -> str:
 
 def build(verbose: bool = True, out: str = OUT, defines: tuple = ()) -> str:
     """Compile and link the library.  ``defines`` set the kernels' tuning
-    macros (CHAMP_MJB, CHAMP_MOVE_WPE, CHAMP_HJB, CHAMP_HJAS_WPE, CHAMP_NL_QB,
+    macros (CHAMP_MOVE_WPE, CHAMP_SWEEP_WPE, CHAMP_MOVE_NW, CHAMP_HJB, CHAMP_HJAS_WPE, CHAMP_NL_QB,
     CHAMP_NL_WPE); ``out`` other than the default builds a variant elsewhere."""
     objdir = OBJDIR if not defines and out == OUT else out + ".objs"
     os.makedirs(objdir, exist_ok=True)

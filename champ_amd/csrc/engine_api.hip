@@ -748,9 +748,10 @@ extern "C" int champ_gpu_accept(champ_ctx *c, int32_t iel, const uint8_t *accept
     return CHAMP_OK;
 }
 
-// One single-electron move of every walker (drift, proposal, ratio, decision,
-// commit) and the periodic refresh of the Slater inverses.
-int launch_move_step(champ_ctx *c, int iel)
+// One single-electron move of every walker of a multideterminant trial function
+// (drift, proposal, ratio, decision, commit) and the periodic refresh of the
+// Slater inverses.
+static int launch_move_step(champ_ctx *c, int iel)
 {
     int rc;
     if ((rc = launch_md_pre_timed(c, iel))) return rc;
@@ -760,6 +761,24 @@ int launch_move_step(champ_ctx *c, int iel)
     if ((rc = launch_move_b(c, iel, 0))) return rc;
     if (c->lu_every > 0 && (iel + 1) % c->lu_every == 0 && iel + 1 < c->NE && (rc = launch_slater_refresh(c)))
         return rc;
+    return CHAMP_OK;
+}
+
+// The moves of a sweep with the context's mover: one launch for a single
+// determinant (split where the inverse is recomputed), else electron by electron.
+int launch_moves(champ_ctx *c)
+{
+    int rc;
+    if (c->md) {
+        for (int iel = 0; iel < c->NE; iel++)
+            if ((rc = launch_move_step(c, iel))) return rc;
+        return CHAMP_OK;
+    }
+    const int step = c->lu_every > 0 ? c->lu_every : c->NE;
+    for (int e = 0; e < c->NE; e += step) {
+        if (e > 0 && (rc = launch_slater_refresh(c))) return rc;
+        if ((rc = launch_sweep_moves(c, e, std::min(c->NE, e + step)))) return rc;
+    }
     return CHAMP_OK;
 }
 
@@ -780,8 +799,7 @@ static int launch_sweep(champ_ctx *c)
 {
     int rc;
     if (c->nloc > 0 && (rc = launch_rotqua(c))) return rc;
-    for (int iel = 0; iel < c->NE; iel++)
-        if ((rc = launch_move_step(c, iel))) return rc;
+    if ((rc = launch_moves(c))) return rc;
     return launch_hpsi_impl(c, 1);
 }
 
@@ -1064,17 +1082,21 @@ extern "C" int champ_gpu_metrop1_batch(champ_ctx *const *ctxs, int32_t n, int32_
     for (int m = 0; m < n; m++) { ctxs[m]->tau = tau; ctxs[m]->imetro = 1; }
     for (int m = 0; m < n; m++) HIPCHECK(hipMemsetAsync(ctxs[m]->esum_dev, 0, sizeof(double) * 4, ctxs[m]->stream));
     // Each population's kernels go to its own stream in the order of its
-    // own metrop1 sweep; the host deals the move steps round-robin over the
-    // populations so that all of them have work queued at once, and queues
-    // a population's hpsi right after its last electron.
+    // own metrop1 sweep; the host deals the move steps of the multideterminant
+    // populations round-robin so that all of them have work queued at once, and
+    // queues a population's hpsi right after its last electron.
     int rc;
     for (int isw = 0; isw < nsweep; isw++) {
-        for (int m = 0; m < n; m++)
-            if (ctxs[m]->nloc > 0 && (rc = launch_rotqua(ctxs[m]))) return rc;
+        for (int m = 0; m < n; m++) {
+            champ_ctx *c = ctxs[m];
+            if (c->nloc > 0 && (rc = launch_rotqua(c))) return rc;
+            // one determinant: the whole sweep in a few launches
+            if (!c->md && ((rc = launch_moves(c)) || (rc = launch_hpsi_impl(c, 1)))) return rc;
+        }
         for (int iel = 0; iel < nemax; iel++)
             for (int m = 0; m < n; m++) {
                 champ_ctx *c = ctxs[m];
-                if (iel >= c->NE) continue;
+                if (iel >= c->NE || !c->md) continue;
                 if ((rc = launch_move_step(c, iel))) return rc;
                 if (iel == c->NE - 1 && (rc = launch_hpsi_impl(c, 1))) return rc;
             }
@@ -1204,7 +1226,7 @@ extern "C" int champ_gpu_basis_fns_noalloc(champ_ctx *c, int32_t npt, const doub
 
 static const char *kclass_name[K_NCLASS] = {"move_jastrow_ao", "move_mo_gemm", "move_ratio_commit", "hpsi_jastrow",
                                             "hpsi_ao", "hpsi_mo_gemm", "hpsi_slater_lu", "hpsi_ecp_prep", "hpsi_nonloc",
-                                            "hpsi_nonloc_psi", "hpsi_eloc", "multidet", "other"};
+                                            "hpsi_nonloc_psi", "hpsi_eloc", "multidet", "moves", "other"};
 
 extern "C" int champ_gpu_kernel_times(champ_ctx *c, int32_t *n, char *names, double *ms, int64_t *launches)
 {

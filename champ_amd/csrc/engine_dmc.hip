@@ -31,8 +31,8 @@
 #include <string>
 #include <vector>
 
-// one single-electron move of every walker with the context's mover (engine_api.hip)
-int launch_move_step(champ_ctx *c, int iel);
+// the moves of every electron of every walker with the context's mover (engine_api.hip)
+int launch_moves(champ_ctx *c);
 int launch_forced_move(champ_ctx *c, int iel);
 
 namespace champ {
@@ -466,9 +466,9 @@ extern "C" int champ_gpu_dmc_step(champ_ctx *c, champ_dmc_step_stats *st)
     HIPCHECK(hipMemsetAsync(c->esum_dev, 0, sizeof(double) * 4, c->stream));
     c->tau = D.tau;
     c->imetro = 2;
-    for (int iel = 0; iel < c->NE; iel++)
-        if ((rc = launch_move_step(c, iel))) { c->imetro = 1; return rc; }
+    rc = launch_moves(c);
     c->imetro = 1;
+    if (rc) return rc;
     const bool tmoves = D.icasula < 0 && c->nloc > 0;
     c->tstore = tmoves ? 1 : 0;
     rc = launch_hpsi_impl(c, 0);

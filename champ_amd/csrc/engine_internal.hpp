@@ -47,7 +47,7 @@ struct Timer {
 };
 
 enum KClass { K_MOVE_A = 0, K_MOVE_GEMM, K_MOVE_B, K_HPSI_JAS, K_HPSI_AO, K_HPSI_GEMM, K_HPSI_SLATER,
-              K_HPSI_ECP, K_HPSI_NONLOC, K_HPSI_PSI, K_HPSI_ELOC, K_MD, K_OTHER, K_NCLASS };
+              K_HPSI_ECP, K_HPSI_NONLOC, K_HPSI_PSI, K_HPSI_ELOC, K_MD, K_SWEEP, K_OTHER, K_NCLASS };
 
 }  // namespace champ
 
@@ -237,6 +237,7 @@ enum { DMC_PP = 0, DMC_DFUS2AC, DMC_DFUS2UN, DMC_PSUM, DMC_NODECR, DMC_IACCEPT, 
 enum { DMC_O_WT = 0, DMC_O_WE, DMC_O_PE, DMC_O_TPB, DMC_O_TAU, DMC_O_PSUM, DMC_O_NODECR, DMC_OUT = 8 };
 // kernel launchers (engine_kernels.hip)
 int launch_move_a(champ_ctx *c, int iel, int mode);
+int launch_sweep_moves(champ_ctx *c, int e0, int e1);  // one determinant: the moves of electrons e0 .. e1 - 1
 int launch_move_gemm(champ_ctx *c);
 int launch_move_b(champ_ctx *c, int iel, int mode);
 int launch_drift_old(champ_ctx *c, int iel);

@@ -17,6 +17,7 @@
 #include <utility>
 
 #define __global__
+#define MOVE_ARGS_AGAIN(a) (a)  // no kernel argument segment here
 #define __device__
 #define __host__
 #define __forceinline__ inline
@@ -126,7 +127,8 @@ inline double __builtin_amdgcn_rsq(double x) { return (1.0 / std::sqrt(x)) * (1.
 inline double __builtin_amdgcn_rcp(double x) { return (1.0 / x) * (1.0 + 0x1p-27); }
 inline void __builtin_amdgcn_sched_barrier(int) {}  // scheduling only
 // Register move between the lanes of a row of 16 by its DPP control word:
-// quad_perm (0x00-0xff), row_mirror (0x140) and row_half_mirror (0x141)
+// quad_perm (0x00-0xff), row_ror (0x121-0x12f), row_mirror (0x140) and
+// row_half_mirror (0x141)
 inline int __builtin_amdgcn_mov_dpp(int v, int ctrl, int, int, bool)
 {
     uint64_t all[64];
@@ -134,6 +136,7 @@ inline int __builtin_amdgcn_mov_dpp(int v, int ctrl, int, int, bool)
     const int l = emu::tctx.lane % 64;
     int src = l;
     if (ctrl < 0x100) src = (l & ~3) | ((ctrl >> (2 * (l & 3))) & 3);
+    else if (ctrl > 0x120 && ctrl < 0x130) src = (l & ~15) | ((l - (ctrl & 15)) & 15);
     else if (ctrl == 0x140) src = (l & ~15) | (15 - (l & 15));
     else if (ctrl == 0x141) src = (l & ~7) | (7 - (l & 7));
     else { fprintf(stderr, "emu: DPP control %x not modelled\n", ctrl); abort(); }

@@ -79,3 +79,46 @@ def test_quadrature_of_shell_sets(require_gpu, heavy, hyd, drop):
         o.set_quad(sy.xq0, sy.yq0, sy.zq0)
         d = o.hpsi()
         assert abs(g["energy"][w] - d["energy"]) <= 1e-9 * max(1.0, abs(d["energy"]), abs(d["ekin"]))
+
+
+# (2, 1, 9): one pass of 16 lanes; 33 and 65 electrons: a full pass and a remainder of 1;
+# 97: 64 + 33 (two passes of 64 lanes); 40: one pass; spins above 32, 80 (five and ten
+# columns of the update) through 65 and 170 electrons
+@pytest.mark.parametrize("shape", [(2, 1, 9, 2, True), (5, 0, 33, 5, True), (9, 4, 65, 4, True), (13, 7, 97, 3, False),
+                                   (6, 2, 40, 4, True), (22, 0, 170, 4, True)], ids=lambda s: "-".join(map(str, s)))
+@pytest.mark.parametrize("nwalk", [3, 1030])
+@pytest.mark.parametrize("mover", [1, 6])
+def test_sweep_of_odd_shapes(require_gpu, shape, nwalk, mover):
+    """One sweep against the oracle's, with few walkers (several wavefronts per
+    walker) and with many (one per walker); the first and last walkers are compared."""
+    if "emu" in ENGINE_LIB and nwalk > 100:
+        pytest.skip("population too large for the host emulation")
+    if mover == 6 and shape[2] > 128:
+        pytest.skip("ill-conditioned start: its small determinant ratios amplify roundings to 1e-7, in any kernel")
+    sy = molecule(*shape)
+    x = sy.initial_walkers(nwalk, seed=6)
+    eng = Engine(sy, nwalk, lib_path=ENGINE_LIB)
+    eng.set_walkers(x)
+    st = np.random.default_rng(5).integers(1, 2 ** 63 - 1, size=(nwalk, 4), dtype=np.uint64)
+    eng.set_rng(st)
+    eng.hpsi()
+    r = eng.metrop1(1, 0.3) if mover == 1 else eng.metrop6(1)
+    assert 0 < r["accepted"] <= r["proposed"]
+    # a proposal outside every AO's cut radius has the ratio 0, which flags the walker (2)
+    assert not np.any(eng.status() & ~2)
+    got, sc, rng = eng.get_walkers(), eng.scalars(), eng.get_rng()
+    for w in (0, 1, nwalk - 1):
+        o = ffi.walker(sy)
+        o.set_x(x[w])
+        o.set_rng(st[w])
+        if sy.nloc:
+            o.set_quad(sy.xq0, sy.yq0, sy.zq0)
+        o.hpsi()
+        o.sweep(0.3) if mover == 1 else o.sweep6()
+        d = o.scalars()
+        # the same decisions, positions to the rounding of the drifts, ln psi and E_L
+        # to that of an inverse updated once per electron
+        assert np.array_equal(rng[w], o.get_rng())
+        assert np.max(np.abs(got[w] - o.get_x())) < 1e-8
+        assert abs(sc["psijo"][w] - d["psijo"]) < 1e-8 * max(1.0, abs(d["psijo"]))
+        assert abs(sc["eold"][w] - d["eold"]) < 1e-6 * max(1.0, abs(d["eold"]))
