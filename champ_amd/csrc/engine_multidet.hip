@@ -225,15 +225,19 @@ __device__ void md_dets(const MdArgs &m, int s, const double *aa, double *D)
     }
 }
 
-__device__ double md_block_sum(double v, double *red)
+// Sum of v over the block's first MD_SUM threads.  A block may have more: which terms
+// meet in a partial sum, and so the rounding that a trajectory would amplify, does not
+// depend on its size.
+constexpr int MD_SUM = 256;
+__device__ double md_block_sum(double v, double *red /*[MD_SUM / WAVE]*/)
 {
-    const int lane = threadIdx.x % WAVE, wv = threadIdx.x / WAVE, nwv = blockDim.x / WAVE;
+    const int lane = threadIdx.x % WAVE, wv = threadIdx.x / WAVE;
     v = wave_sum(v);
     __syncthreads();
-    if (lane == 0) red[wv] = v;
+    if (lane == 0 && wv < MD_SUM / WAVE) red[wv] = v;
     __syncthreads();
     double t = 0;
-    for (int i = 0; i < nwv; i++) t += red[i];
+    for (int i = 0; i < MD_SUM / WAVE; i++) t += red[i];
     __syncthreads();
     return t;  // on every thread
 }
@@ -242,7 +246,9 @@ __device__ double md_block_sum(double v, double *red)
 __device__ double md_sum(const MdArgs &m, const double *Dup, const double *Ddn, double *red)
 {
     double s = 0;
-    for (int k = threadIdx.x; k < m.ndet; k += blockDim.x) s += m.cdet[k] * Dup[m.du[k]] * Ddn[m.dd[k]];
+    if (threadIdx.x < MD_SUM)
+#pragma unroll 8  // eight terms' gathers in flight
+        for (int k = threadIdx.x; k < m.ndet; k += MD_SUM) s += m.cdet[k] * Dup[m.du[k]] * Ddn[m.dd[k]];
     return md_block_sum(s, red);
 }
 
@@ -258,7 +264,9 @@ __device__ void md_weights(const MdArgs &m, int w, int s, const double *Do, doub
     const int *oth = m.woth[s];
     for (int u = threadIdx.x; u < m.nu[s]; u += blockDim.x) {
         double t = 0;
-        for (int e = m.woff[s][u]; e < m.woff[s][u + 1]; e++) t += cf[e] * Do[oth[e]];
+        const int e1 = m.woff[s][u + 1];
+#pragma unroll 8
+        for (int e = m.woff[s][u]; e < e1; e++) t += cf[e] * Do[oth[e]];
         Wt[u] = t * sinv;
     }
     __syncthreads();
@@ -322,7 +330,9 @@ __device__ void md_zgather(const MdArgs &m, int w, int s, double scale, double *
     const int lane = threadIdx.x % WAVE, wv = threadIdx.x / WAVE, nwv = blockDim.x / WAVE;
     for (int v = wv; v < m.nv[s]; v += nwv) {
         double x = 0;
-        for (int e = m.zoff[s][v] + lane; e < m.zoff[s][v + 1]; e += WAVE) {
+        const int e1 = m.zoff[s][v + 1];
+#pragma unroll 4
+        for (int e = m.zoff[s][v] + lane; e < e1; e += WAVE) {
             const int ent = m.zent[s][e];
             x += Wt[ent >> 2] * tb[ent];
         }
@@ -337,7 +347,7 @@ __device__ void md_zgather(const MdArgs &m, int w, int s, double scale, double *
 // from V; one block per walker of the current chunk (orbitals in orball).
 __global__ void __launch_bounds__(256) k_md_hpsi(MdArgs m)
 {
-    __shared__ double red[8];
+    __shared__ double red[MD_SUM / WAVE];
     const int wc = blockIdx.x, w = m.w0 + wc, tid = threadIdx.x, bd = blockDim.x;
     const int NE = m.NE, NO = m.NO, NV = m.NV, NM = m.NM;
     const double *ob = m.orball + (size_t)wc * NE * 5 * NO;
@@ -405,9 +415,17 @@ __global__ void __launch_bounds__(256) k_md_hpsi(MdArgs m)
     }
 }
 
+// threads of a block of the per-move kernels at most
+constexpr int MD_MOVE_THREADS = 512;
+
 // ------------------------------------------------------------------------
 // Column iel of V at the current configuration (drift at the old position).
-__global__ void __launch_bounds__(256) k_md_pre(MdArgs m)
+// Bound by the latency of the gathers: a weight or a sum of determinants is a chain of
+// additions whose operands come through an index each.  The chains keep their order (a
+// trajectory amplifies a rounding); eight terms' gathers are in flight instead of one:
+// 256 electrons, 5000 determinants, 384 walkers 324 -> 159 us a kernel of the pair, a
+// DMC step of 500 determinants, 1536 walkers 4.22 -> 3.51 ms.
+__global__ void __launch_bounds__(MD_MOVE_THREADS) k_md_pre(MdArgs m)
 {
     const int w = blockIdx.x, tid = threadIdx.x, bd = blockDim.x;
     const int NE = m.NE, NO = m.NO, NV = m.NV, NM = m.NM, iel = m.iel;
@@ -430,6 +448,7 @@ __global__ void __launch_bounds__(256) k_md_pre(MdArgs m)
         double x = 0;
         if (j >= 0) {
             double c = 0;
+#pragma unroll 8
             for (int vv = 0; vv < nv; vv++) c += aa[(size_t)j * NV + vv] * z[vv];
             x = A[(size_t)i * NM + j] - c;
         } else if (v >= 0) {
@@ -444,9 +463,9 @@ __global__ void __launch_bounds__(256) k_md_pre(MdArgs m)
 // determinants and cofactors into the spare buffer, S' and column iel of the
 // new V (drift at the new position).  The reference ratio R0 = 0 leaves S' = 0
 // (psi_D' = 0: the move is refused and the walker flagged by the ratio kernel).
-__global__ void __launch_bounds__(256) k_md_post(MdArgs m)
+__global__ void __launch_bounds__(MD_MOVE_THREADS) k_md_post(MdArgs m)
 {
-    __shared__ double red[8];
+    __shared__ double red[MD_SUM / WAVE];
     const int w = blockIdx.x, tid = threadIdx.x, bd = blockDim.x;
     const int NE = m.NE, NO = m.NO, NV = m.NV, NM = m.NM, iel = m.iel;
     const int s = iel < m.NUP ? 0 : 1, nel = s ? NE - m.NUP : m.NUP, ish = s ? m.NUP : 0, i = iel - ish;
@@ -455,7 +474,8 @@ __global__ void __launch_bounds__(256) k_md_post(MdArgs m)
     const double *on = m.orbn + (size_t)w * 4 * NO;
     const int *ko = m.iworbd + ish;
     double r0 = 0;
-    for (int j = tid; j < nel; j += bd) r0 += A[(size_t)i * NM + j] * on[ko[j]];
+    if (tid < MD_SUM)
+        for (int j = tid; j < nel; j += MD_SUM) r0 += A[(size_t)i * NM + j] * on[ko[j]];
     const double R0 = md_block_sum(r0, red);
     double *vcn = m.vcoln + (size_t)w * NO;
     if (R0 == 0.0) {
@@ -468,6 +488,7 @@ __global__ void __launch_bounds__(256) k_md_post(MdArgs m)
     double *gw = m.g + (size_t)w * NV;
     for (int v = tid; v < nv; v += bd) {
         double x = on[m.virt[s][v]];
+#pragma unroll 8
         for (int j = 0; j < nel; j++) x -= on[ko[j]] * aa[(size_t)j * NV + v];
         gw[v] = x;
     }
@@ -505,6 +526,7 @@ __global__ void __launch_bounds__(256) k_md_post(MdArgs m)
         double x = 0;
         if (j >= 0) {
             double c = 0;
+#pragma unroll 8
             for (int vv = 0; vv < nv; vv++) c += aar[(size_t)j * NV + vv] * z[vv];
             x = A[(size_t)i * NM + j] * rinv - c;
         } else if (v >= 0) {
@@ -537,12 +559,27 @@ static MdArgs md_move_args(champ_ctx *c, int iel, size_t *lds)
     return m;
 }
 
+#ifndef CHAMP_MD_THREADS  // variant builds: fixed threads per block
+#define CHAMP_MD_THREADS 0
+#endif
+
+// Threads of a walker's block in the per-move kernels: 512 where the walkers leave
+// wavefront slots free and there are more than 256 unique determinants to take them,
+// else 256.  ms of the kernels in a sweep with 256 / 512 / 1024 threads: 256 electrons,
+// 5000 determinants, 384 walkers 81.9 / 72.3 / 107.1; 22 electrons, 60 determinants, 2000
+// walkers 1.35 / 1.90 / 3.09; a DMC step of 500 determinants, 1536 walkers 3.51 / 4.28 / 5.64.
+static int md_threads(const champ_ctx *c)
+{
+    if (CHAMP_MD_THREADS) return CHAMP_MD_THREADS;
+    return c->W <= 512 && std::max(c->md_nu[0], c->md_nu[1]) > 256 ? 512 : 256;
+}
+
 int launch_md_pre(champ_ctx *c, int iel)
 {
     if (!c->md) return CHAMP_OK;
     size_t lds;
     const MdArgs m = md_move_args(c, iel, &lds);
-    hipLaunchKernelGGL(k_md_pre, dim3(c->W), dim3(256), lds, c->stream, m);
+    hipLaunchKernelGGL(k_md_pre, dim3(c->W), dim3(md_threads(c)), lds, c->stream, m);
     HIPCHECK(hipGetLastError());
     return CHAMP_OK;
 }
@@ -552,7 +589,7 @@ int launch_md_post(champ_ctx *c, int iel)
     if (!c->md) return CHAMP_OK;
     size_t lds;
     const MdArgs m = md_move_args(c, iel, &lds);
-    hipLaunchKernelGGL(k_md_post, dim3(c->W), dim3(256), lds, c->stream, m);
+    hipLaunchKernelGGL(k_md_post, dim3(c->W), dim3(md_threads(c)), lds, c->stream, m);
     HIPCHECK(hipGetLastError());
     return CHAMP_OK;
 }
