@@ -598,7 +598,9 @@ __global__ void __launch_bounds__(MMA_THREADS) CHAMP_WAVES_PER_EU(CHAMP_MMA_WPE)
         __syncthreads();
 
         // ---- points: x_qb, the e-n sums and the parts of the e-e-n sum that
-        // hold one point-centre distance (X_k; the k = 0 terms)
+        // hold one point-centre distance (X_k; the k = 0 terms), in FP64 on both
+        // paths: they weigh a whole point, X_k times the sum of its u^k over the
+        // partners (13.3 ms of 160 electrons x 4096 walkers in FP64, 12.8 in FP32)
         {
             const int pt = tid % MMA_MP, tg = tid / MMA_MP;
             double sen = 0.0, sx[NP];
@@ -611,22 +613,22 @@ __global__ void __launch_bounds__(MMA_THREADS) CHAMP_WAVES_PER_EU(CHAMP_MMA_WPE)
                 const double px = live ? XP[3 * pt] : 0.0, py = live ? XP[3 * pt + 1] : 0.0;
                 const double pz = live ? XP[3 * pt + 2] : 0.0;
                 for (int b = tg; b < NC; b += MMA_TG) {
-                    T xq = T(0);
+                    double xq = 0.0;
                     if (live) {
-                        const T e0 = (T)(px - a.cent[3 * b]), e1 = (T)(py - a.cent[3 * b + 1]), e2 = (T)(pz - a.cent[3 * b + 2]);
-                        T r2 = 0;
+                        const double e0 = px - a.cent[3 * b], e1 = py - a.cent[3 * b + 1], e2 = pz - a.cent[3 * b + 2];
+                        double r2 = 0;
                         r2 = r2 + e0 * e0; r2 = r2 + e1 * e1; r2 = r2 + e2 * e2;
-                        const T rq = b == ic ? (T)a.r_en[((size_t)w * NC + ic) * NE + i] : sqrt_inner(r2);
-                        xq = exp_neg((T)(-kapd * (double)rq));
-                        const T rr = (T(1) - xq) * (T)jp.asymp_r;
-                        sen += (double)en_term<T>(jp, sT[b], rr, xq);
+                        const double rq = b == ic ? a.r_en[((size_t)w * NC + ic) * NE + i] : sqrt_inner(r2);
+                        xq = exp_neg(-kapd * rq);
+                        const double rr = (1.0 - xq) * jp.asymp_r;
+                        sen += en_term<double>(jp, sT[b], rr, xq);
                         double xp[NORDC + 1];
-                        een_powers<NORDC>((double)xq, xp);
+                        een_powers<NORDC>(xq, xp);
                         een_uncoupled<NORDC>(jp.c[sT[b]], xp, sx);
 #pragma unroll
                         for (int n = 1; n <= NP; n++) sen += xp[n] * D0[((size_t)p * NP + n - 1) * NC + b];
                     }
-                    XQ[(size_t)b * MMA_MP + pt] = xq;
+                    XQ[(size_t)b * MMA_MP + pt] = (T)xq;
                 }
                 TP[tg * MMA_MP + pt] = sen;
 #pragma unroll
