@@ -40,7 +40,7 @@ __global__ void __launch_bounds__(256) k_drift_old(MoveArgs a)
 //   writing the AO block that the MO GEMM contracts (orbitalse).
 // The sweeps of one determinant take k_sweep (engine_sweep.hip) instead.
 // A wavefront per 64 partners instead of one per walker: 256 electrons x 384
-// walkers 188 -> 92 us.
+// walkers 188 -> 73 us.
 #ifndef CHAMP_MOVE_WPE  // waves per SIMD asked of the register allocator
 #define CHAMP_MOVE_WPE 1
 #endif

@@ -136,6 +136,104 @@ __device__ __forceinline__ void sm_update(double *S, int NM, int nel, int row, d
     }
 }
 
+// Orbitals of the moved electrons' spin, value and gradient, into orb_b [walker][4]
+// [npad]: the AOs a chunk of 64 NW at a time through LDS against the occupied
+// coefficients ct [nel][NB], tiles of 16 orbitals dealt to the wavefronts.  Four
+// walkers x four components fill the 16 rows of an instruction and share every
+// coefficient read; a block of one walker runs on the 4 x 4 x 4 form, four blocks of
+// it for 16 orbitals (17 cycles; on the 16-row form, a quarter of it used, 66: 11.1
+// against 10.0 ms of moves a sweep of 160 electrons x 256 walkers).  Four walkers a
+// wavefront each on the 4 x 4 x 4 form read the coefficients four times: 2.59 against
+// 2.36 ms at 60 electrons x 768 walkers.  Both forms add the four products of a step in
+// order, and steps pair them as k_gemm_mfma.  The coefficients of the next KS AOs
+// are loaded while these run.
+template <int NORDC, typename T, int NW>
+__device__ __forceinline__ void sweep_orbitals(const MoveArgs &a, const MoveLds<NORDC, T> &L, bool live, const double *ct,
+                                               int nel, int npad, int bt, int wpb, double *chunks, double *orb_b)
+{
+    constexpr int NT = NW * WAVE, KS = NW > 1 ? 64 : 32, TC = 2, SPC = NT / KS;  // TC tiles at a time
+    const int NB = a.NB, nt = (nel + 15) / 16, stride = SweepLds<NORDC, T, NW>::stride(wpb);
+    const int r = bt % 16, q = (bt % WAVE) / 16, wvb = bt / WAVE, nwb = blockDim.x / WAVE, wb = bt / NT, tid = bt % NT;
+    const bool rows16 = NW == 1 && wpb == 4;
+    for (int t0 = wvb; t0 - wvb < nt; t0 += TC * nwb) {
+        dbl4 acc16[TC];
+        double acc4[TC], b0[TC][KS / 4], b1[TC][KS / 4];
+#pragma unroll
+        for (int i = 0; i < TC; i++) { acc16[i] = dbl4{0.0, 0.0, 0.0, 0.0}; acc4[i] = 0.0; }
+        auto load = [&](int k0, double (*b)[KS / 4]) {
+#pragma unroll
+            for (int i = 0; i < TC; i++) {
+                const int t = t0 + i * nwb, col = 16 * t + r;
+                if (t >= nt) continue;
+                const double *cp = ct + (size_t)(col < nel ? col : 0) * NB + 4 * q;
+                if (k0 + KS <= NB) {
+#pragma unroll
+                    for (int k = 0; k < KS / 4; k++) b[i][k] = cp[k0 + 16 * (k / 4) + k % 4];
+                } else {
+#pragma unroll
+                    for (int k = 0; k < KS / 4; k++) {
+                        const int kk = k0 + 16 * (k / 4) + k % 4;
+                        b[i][k] = kk + 4 * q < NB ? cp[kk] : 0.0;
+                    }
+                }
+            }
+        };
+        auto mma = [&](const double *A, const double (*b)[KS / 4]) {  // A: the chunk from the stage's first AO
+            if (rows16) {
+#pragma unroll
+                for (int k = 0; k < KS / 4; k++) {
+                    const double av = A[(size_t)(16 * (k / 4) + 4 * q + k % 4) * stride + r];
+#pragma unroll
+                    for (int i = 0; i < TC; i++)
+                        if (t0 + i * nwb < nt) acc16[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, b[i][k], acc16[i], 0, 0, 0);
+                }
+            } else {
+#pragma unroll
+                for (int k = 0; k < KS / 4; k++) {
+                    const double av = A[(size_t)(16 * (k / 4) + 4 * q + k % 4) * stride + 4 * wb + r % 4];
+#pragma unroll
+                    for (int i = 0; i < TC; i++)
+                        if (t0 + i * nwb < nt) acc4[i] = __builtin_amdgcn_mfma_f64_4x4x4f64(av, b[i][k], acc4[i], 0, 0, 0);
+                }
+            }
+        };
+        load(0, b0);
+        int buf = 0;
+        for (int m0 = 0; m0 < NB; m0 += NT, buf ^= 1) {
+            double *A = chunks + (size_t)buf * NT * stride;
+            const int m = m0 + tid;
+            T out[5] = {T(0), T(0), T(0), T(0), T(0)};
+            if (live && m < NB) move_ao(L, a.ao_cent[m], a.ao_ri[m], a.ao_slm[m], out);
+#pragma unroll
+            for (int k = 0; k < 4; k++) A[(size_t)tid * stride + 4 * wb + k] = (double)out[k];
+            if (nwb > 1) __syncthreads();  // the other buffer was read before the last one
+            else __syncwarp();
+#pragma unroll
+            for (int st = 0; st < SPC; st += 2) {
+                const int k0 = m0 + st * KS;
+                if (k0 + KS < NB) load(k0 + KS, b1);
+                if (k0 < NB) mma(A + (size_t)st * KS * stride, b0);
+                if (k0 + 2 * KS < NB) load(k0 + 2 * KS, b0);
+                if (k0 + KS < NB) mma(A + (size_t)(st + 1) * KS * stride, b1);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < TC; i++) {
+            const int t = t0 + i * nwb;
+            if (t >= nt) continue;
+            if (rows16) {
+#pragma unroll
+                for (int v = 0; v < 4; v++)  // rows 4 v + q: component q of the block's walker v
+                    orb_b[(size_t)(4 * v + q) * npad + 16 * t + r] = acc16[i][v];
+            } else {
+                orb_b[(size_t)(4 * wb + q) * npad + 16 * t + r] = acc4[i];
+            }
+        }
+        if (nwb > 1) __syncthreads();  // the chunks are written again
+        else __syncwarp();
+    }
+}
+
 // ------------------------------------------------------------------------
 // One determinant: the moves of electrons e0 .. e1 - 1 of every walker in one
 // launch.  Walkers do not meet inside a sweep, so a block takes its walkers
@@ -146,18 +244,14 @@ __device__ __forceinline__ void sm_update(double *S, int NM, int nel, int row, d
 // decision) overlaps other walkers' sums.
 //   NW = 1: a wavefront per walker, up to four walkers to a block; NW = 4: a block
 //   per walker.
-// The orbitals: the block's AOs go a chunk at a time through LDS as the rows
-// (walker, component) of a matrix product with the occupied coefficients, 16
-// orbitals per tile and the tiles dealt to the wavefronts; four walkers fill the
-// instruction's 16 rows and share every coefficient read.  Products are paired
-// and added as in k_gemm_mfma, the drift, ratio and update as in k_move_b, so a
-// sweep gives the bits of the separate kernels.
+// Sums keep the order of the separate kernels (k_move_a, k_gemm_mfma, k_move_b), so a
+// sweep gives their bits.
 // ms of a sweep's moves, as three launches per electron (Jastrow and AOs, matrix
-// product, decision and commit) and so: 160 electrons x 4096 walkers 90.3 -> 68.7
-// (mixed 72.9 -> 54.8), x 1024 33.3 -> 23.8, x 256 27.2 -> 11.1; 60 x 768 5.0 ->
-// 2.36; 22 x 256 1.15 -> 0.51; 10 x 4 0.41 -> 0.18.  Few walkers: the chains of one
-// move (7 us of serial head, one lane's sum over the centres); many: two waves per
-// SIMD (256 registers of the pair loop) on the FP64 pipe, and the commit's columns.
+// product, decision and commit) and so: 160 electrons x 4096 walkers 90.3 -> 57.5
+// (mixed 72.9 -> 51.0), x 256 27.2 -> 8.4; 60 x 768 5.0 -> 2.2; 22 x 256 1.15 -> 0.49;
+// 10 x 4 0.41 -> 0.17.  Few walkers: the chains of one move (of 10 us at 10 electrons 4
+// are the proposal's and 3 the decision's scalar code); many: the pair loop, two waves
+// per SIMD of its 207 registers, on the FP64 pipe and on its 16 bytes per pair and centre.
 template <int NORDC, typename T, int NW, int MOVERS>
 __global__ void __launch_bounds__(SW_BLOCK) CHAMP_WAVES_PER_EU(CHAMP_SWEEP_WPE) k_sweep(MoveArgs args, int e0, int e1)
 {
@@ -257,65 +351,7 @@ __global__ void __launch_bounds__(SW_BLOCK) CHAMP_WAVES_PER_EU(CHAMP_SWEEP_WPE) 
             team_sync<BLOCK>();
             if (BLOCK) { psijn = s_sum[0]; for (int k = 0; k < 3; k++) vjn[k] = s_sum[1 + k]; }
         }
-        // ---- orbitals of the moved electrons' spin, value and gradient
-        {
-            const int stride = SL::stride(wpb), nt = (nel + 15) / 16, nwb = blockDim.x / WAVE, wvb = bt / WAVE, NB = a.NB;
-            const double *ct = a.cocc[iab];
-            const int r = bt % 16, q = (bt % WAVE) / 16;
-            const bool rok = r < 4 * wpb;
-            for (int t0 = 0; t0 < nt; t0 += 2 * nwb) {  // two tiles per wavefront at a time
-                dbl4 acc[2] = {dbl4{0.0, 0.0, 0.0, 0.0}, dbl4{0.0, 0.0, 0.0, 0.0}};
-                const double *cp[2];
-#pragma unroll
-                for (int i = 0; i < 2; i++) {
-                    const int col = (t0 + wvb + i * nwb) * 16 + r;
-                    cp[i] = ct + (size_t)(col < nel ? col : 0) * NB;
-                }
-                int buf = 0;
-                for (int m0 = 0; m0 < NB; m0 += NT, buf ^= 1) {
-                    double *A = chunks + (size_t)buf * NT * stride;
-                    const int m = m0 + tid;
-                    T out[5] = {T(0), T(0), T(0), T(0), T(0)};
-                    if (live && m < NB) move_ao(L, a.ao_cent[m], a.ao_ri[m], a.ao_slm[m], out);
-#pragma unroll
-                    for (int k = 0; k < 4; k++) A[(size_t)tid * stride + 4 * wb + k] = (double)out[k];
-                    if (blockDim.x > WAVE) __syncthreads();  // the other buffer was read before the last one
-                    else __syncwarp();
-                    const int kn = min(NT, NB - m0);
-                    for (int k0 = 0; k0 < kn; k0 += 16) {
-                        double av[4], bv[2][4];
-#pragma unroll
-                        for (int i = 0; i < 2; i++) {
-                            if (t0 + wvb + i * nwb >= nt) break;
-#pragma unroll
-                            for (int s = 0; s < 4; s++) {
-                                const int k = m0 + k0 + 4 * q + s;
-                                bv[i][s] = k < NB ? cp[i][k] : 0.0;
-                            }
-                        }
-#pragma unroll
-                        for (int s = 0; s < 4; s++) av[s] = rok ? A[(size_t)(k0 + 4 * q + s) * stride + r] : 0.0;
-#pragma unroll
-                        for (int i = 0; i < 2; i++) {
-                            if (t0 + wvb + i * nwb >= nt) break;
-#pragma unroll
-                            for (int s = 0; s < 4; s++)
-                                acc[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[s], bv[i][s], acc[i], 0, 0, 0);
-                        }
-                    }
-                }
-#pragma unroll
-                for (int i = 0; i < 2; i++) {
-                    const int t = t0 + wvb + i * nwb;
-                    if (t >= nt) break;
-#pragma unroll
-                    for (int v = 0; v < 4; v++)  // rows 4 v + q: component q of the block's walker v
-                        if (v < wpb) orb_b[(size_t)(4 * v + q) * npad + 16 * t + r] = acc[i][v];
-                }
-                if (blockDim.x > WAVE) __syncthreads();  // the chunks are written again
-                else __syncwarp();
-            }
-        }
+        sweep_orbitals<NORDC, T, NW>(a, L, live, a.cocc[iab], nel, npad, bt, wpb, chunks, orb_b);
         if (!live) continue;
         // ---- determinant ratio, drift at the proposal, decision
         if (wv == 0) {
@@ -402,9 +438,9 @@ static inline int nblocks(int n, int per) { return (n + per - 1) / per; }
 // Threads per block of single-wavefront walkers.  Up to 512 walkers a block each, so
 // that they spread over the CUs; above, four share the coefficient reads and fill the
 // matrix instruction.  ms of a sweep's moves in blocks of one / four walkers:
-//   electrons 10, walkers 4     0.18 / 0.23    electrons 60, walkers 768  2.43 / 2.36
-//   22, 256                     0.51 / 0.57    160, 1024                  36.5 / 23.8
-//   60, 256                     2.05 / 2.07    160, 4096                  119.6 / 68.7
+//   electrons 10, walkers 4     0.18 / 0.23    electrons 60, walkers 768  2.42 / 2.37
+//   22, 256                     0.53 / 0.58    160, 1024                  31.4 / 24.4
+//   60, 256                     2.06 / 2.07    160, 4096                  105.9 / 69.7
 static int one_wave_block(const champ_ctx *c)
 {
     if (CHAMP_SWEEP_BLOCK) return CHAMP_SWEEP_BLOCK;
@@ -415,10 +451,10 @@ static int one_wave_block(const champ_ctx *c)
 // resident at once (two on a CU, 512) and a move has the work for them, and where the
 // LDS of a block of single-wavefront walkers is too large; else one, which does
 // without barriers.  ms of a sweep's moves with one / four:
-//   electrons 10, walkers 4     0.18 / 0.19    electrons 160, walkers 256  22.2 / 11.1
-//   22, 256                     0.51 / 0.51    160, 1024                   23.8 / 26.1
-//   60, 256                     2.05 / 1.76    160, 4096                   68.7 / 102.7
-//   60, 768                     2.36 / 3.93
+//   electrons 10, walkers 4     0.18 / 0.18    electrons 160, walkers 256  22.2 / 10.0
+//   22, 256                     0.51 / 0.50    160, 1024                   24.4 / 23.3
+//   60, 256                     2.06 / 1.70    160, 4096                   69.7 / 91.9
+//   60, 768                     2.37 / 3.70
 template <int N, typename T>
 static bool one_wave(const champ_ctx *c)
 {

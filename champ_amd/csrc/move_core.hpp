@@ -13,13 +13,14 @@
 
 namespace champ {
 
-// centres whose partner distances are loaded one group ahead: 4 on the FP64
-// path (0.30 against 0.335 ms per move at 160 e x 4096 walkers), 1 on the FP32
-// path (its register budget; 4 ran at 0.32 against 0.24 ms)
+// Centres whose partner distances are in flight.  A ring, each value loaded again as it
+// is taken, waits for one load where a group of centres loaded together waited for all of
+// them: 69.7 -> 57.3 ms of moves a sweep of 160 electrons x 4096 walkers, 55.6 -> 51.0 on
+// the FP32 path (one centre ahead there), 9.8 -> 8.4 at 256 walkers.  Eight give 55.7,
+// 50.7 and 8.8.
 #ifndef CHAMP_MOVE_PF
 #define CHAMP_MOVE_PF 4
 #endif
-template <typename T> constexpr int move_pf() { return sizeof(T) == sizeof(double) ? CHAMP_MOVE_PF : 1; }
 
 // Barrier of the wavefronts that share a walker: the block, or one wavefront.
 template <bool BLOCK>
@@ -111,7 +112,7 @@ __device__ __forceinline__ void move_pair(const MoveGeo &g, const MoveLds<N, T> 
                                           double xn1, double xn2, const double *rw, const double *rrw, const float2 *ew,
                                           int j, bool on, double &f, double gi[3], double gj[3])
 {
-    constexpr int NA = een_naz<N>(), PF = move_pf<T>();
+    constexpr int NA = een_naz<N>(), PF = CHAMP_MOVE_PF;
     constexpr bool F32 = sizeof(T) == sizeof(float);
     const int NE = g.NE, NC = g.NC, iel = g.iel;
     const JasParams &jp = *g.jas;
@@ -159,39 +160,30 @@ __device__ __forceinline__ void move_pair(const MoveGeo &g, const MoveLds<N, T> 
         }
     }
     if constexpr (N > 1) {
-        // distances of the partners to the centres, PF centres at a time with the
-        // next group's loads in flight (lanes past NE read electron 0)
-        double rjc[PF], rrjc[PF], rjn[PF], rrjn[PF];
-        float2 ejc[PF], ejn[PF];
-#pragma unroll
-        for (int p = 0; p < PF; p++) {
-            const int c = p < NC ? p : 0;
+        // distances of the partners to the centres, loaded PF centres ahead into a ring
+        // (lanes past NE read electron 0)
+        double rn[PF], rrn[PF];
+        float2 en[PF];
+        auto load = [&](int p, int c) {
             if constexpr (F32) {
-                ejn[p] = ew[(size_t)c * NE + jq];
+                en[p] = ew[(size_t)c * NE + jq];
             } else {
-                rjn[p] = rw[(size_t)c * NE + jq];
-                rrjn[p] = rrw[(size_t)c * NE + jq];
+                rn[p] = rw[(size_t)c * NE + jq];
+                rrn[p] = rrw[(size_t)c * NE + jq];
             }
-        }
-        for (int c0 = 0; c0 < NC; c0 += PF) {
+        };
 #pragma unroll
-            for (int p = 0; p < PF; p++) {
-                const int cn = c0 + PF + p;
-                if constexpr (F32) {
-                    ejc[p] = ejn[p];
-                    if (cn < NC) ejn[p] = ew[(size_t)cn * NE + jq];
-                } else {
-                    rjc[p] = rjn[p]; rrjc[p] = rrjn[p];
-                    if (cn < NC) {
-                        rjn[p] = rw[(size_t)cn * NE + jq];
-                        rrjn[p] = rrw[(size_t)cn * NE + jq];
-                    }
-                }
-            }
+        for (int p = 0; p < PF; p++) load(p, p < NC ? p : 0);
+        for (int c0 = 0; c0 < NC; c0 += PF) {
 #pragma unroll
             for (int p = 0; p < PF; p++) {
                 const int c = c0 + p;
                 if (c >= NC) break;
+                double rjc = 0, rrjc = 0;
+                float2 ejc = make_float2(0.0f, 0.0f);
+                if constexpr (F32) ejc = en[p];
+                else { rjc = rn[p]; rrjc = rrn[p]; }
+                if (c + PF < NC) load(p, c + PF);
                 const T *tab = L.tab + (size_t)c * 2 * NA;
                 const double rrm = L.rr[c];
                 const T fmf = (T)L.fm[c];
@@ -200,19 +192,19 @@ __device__ __forceinline__ void move_pair(const MoveGeo &g, const MoveLds<N, T> 
                 if (!on) continue;
                 T swj;
                 if constexpr (F32) {
-                    swj = ejc[p].x;
+                    swj = ejc.x;
                     if (rrm == asymp_r && swj == 0.0f) continue;
                 } else {
-                    if (rrm == asymp_r && rrjc[p] == asymp_r) continue;
-                    swj = (T)(1.0 - kap * rrjc[p]);
+                    if (rrm == asymp_r && rrjc == asymp_r) continue;
+                    swj = (T)(1.0 - kap * rrjc);
                 }
                 const EenOut<T> e = een_eval_tab<N, 1, T>(tab, dd1, swj);
                 fs += e.f;
                 sfu += e.fu;
                 const T fmv = e.fx * fmf;
                 T fot;
-                if constexpr (F32) fot = e.fy * ejc[p].y;
-                else fot = e.fy * (-tkap * swj) / (T)rjc[p];
+                if constexpr (F32) fot = e.fy * ejc.y;
+                else fot = e.fy * (-tkap * swj) / (T)rjc;
                 gm[0] += fmv * rvm0; gm[1] += fmv * rvm1; gm[2] += fmv * rvm2;
                 go[0] += fot * (xj[0] - cx); go[1] += fot * (xj[1] - cy);
                 go[2] += fot * (xj[2] - cz);

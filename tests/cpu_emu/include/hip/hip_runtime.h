@@ -178,6 +178,25 @@ inline dbl4 __builtin_amdgcn_mfma_f64_16x16x4f64(double a, double b, dbl4 c, int
     }
     return c;
 }
+// FP64 MFMA 4x4x4, four blocks: lane l supplies A[i = l % 4][k = l / 16] of block
+// (l / 4) % 4 and B[k = l / 16][j = l % 4] of the same block, and holds D[i = l / 16][j
+// = l % 4] of it (measured on gfx950 with a one-hot probe)
+inline double __builtin_amdgcn_mfma_f64_4x4x4f64(double a, double b, double c, int, int, int)
+{
+    uint64_t ua, ub, all_a[64], all_b[64];
+    memcpy(&ua, &a, 8);
+    memcpy(&ub, &b, 8);
+    emu::wave_exchange(ua, all_a);
+    emu::wave_exchange(ub, all_b);
+    const int l = emu::tctx.lane % 64, blk = (l / 4) % 4;
+    for (int k = 0; k < 4; k++) {
+        double x, y;
+        memcpy(&x, &all_a[16 * k + 4 * blk + l / 16], 8);
+        memcpy(&y, &all_b[16 * k + l % 16], 8);
+        c += x * y;
+    }
+    return c;
+}
 // FP32 MFMA 16x16x4: A and B as above; accumulator element r of lane l holds
 // D[4 (l / 16) + r][l % 16] (measured on gfx950 likewise)
 struct flt4 {
