@@ -221,13 +221,16 @@ def per_kernel(sy, W, kt, nxq, path, acc):
     valu = "fp32-valu-unpacked" if path == "mixed" else "fp64-valu"
     mfma = "fp32-mfma" if path == "mixed" else "fp64-mfma"
     work = {
+        "moves": (W * ne * (flops_move_jastrow(ne, nc, nt, nb, nrad) + 8.0 * ns * nb + acc * 4.0 * ns * ns), valu, "TFLOP/s",
+                  "reference count per move and walker: (Ne-1) Nc (25T+60) + AO, 8 Nsigma Nao, 4 Nsigma^2 per accepted",
+                  False),
         "move_jastrow_ao": (W * flops_move_jastrow(ne, nc, nt, nb, nrad), valu, "TFLOP/s",
                             "reference count (Ne-1) Nc (25T+60) + AO per walker", False),
         "move_mo_gemm": (2.0 * 4 * W * no * nb, "fp64-mfma", "TFLOP/s", "2 (4W) norb Nao", True),
         "move_ratio_commit": (W * 8.0 * (ns + 4 * no + 3 * ne) + W * acc * (16.0 * ns * ns + 8.0 * (3 * no + 20 * ne + 2 * nc)),
                               "hbm", "GB/s", "inverse row + orbitals per walker; inverse read+write and the "
                               "Jastrow/orbital commits per accepted walker", True),
-        "hpsi_jastrow": (W * 0.5 * ne * (ne - 1) * nc * (54 * nt + 80), valu, "TFLOP/s",
+        "hpsi_jastrow": (W * 0.5 * ne * (ne - 1) * nc * (54 * nt + 80), "fp64-valu", "TFLOP/s",
                          "reference count Ne(Ne-1)/2 Nc (54T+80) per walker", False),
         "hpsi_mo_gemm": (2.0 * wchunk * ne * 5 * no * nb, "fp64-mfma", "TFLOP/s", "2 (5 Ne W_chunk) norb Nao", True),
         "hpsi_slater_lu": (wchunk * 2 * 2.0 * ns ** 3, "fp64-valu", "TFLOP/s", "2 Nsigma^3 per spin matrix", True),
