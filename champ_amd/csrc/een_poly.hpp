@@ -95,14 +95,16 @@ constexpr int een_naz() { return EenTable<N>{}.naz > 0 ? EenTable<N>{}.naz : 1; 
 
 // Coefficient tables of one (electron, centre) at switched distance x:
 // tab[d * naz + idx] = d^d A / dx^d for d = 0..D.  c = parameters of the
-// centre's type in term order.
-template <int N, int D, typename T = double>
-__device__ __forceinline__ void een_tables(const double *c, T x, T *tab)
+// centre's type in term order.  C: the type they are formed in; FP32 tables of
+// pair sums are formed in FP64 and rounded once, since a rounded parameter would
+// shift every pair the same way.
+template <int N, int D, typename T = double, typename C = T>
+__device__ __forceinline__ void een_tables(const double *c, C x, T *tab)
 {
     constexpr EenTable<N> ET{};
     constexpr int NA = een_naz<N>();
-    T xp[N + 1];
-    xp[0] = T(1);
+    C xp[N + 1];
+    xp[0] = C(1);
 #pragma unroll
     for (int p = 1; p <= N; p++) xp[p] = p == 1 ? x : xp[1] * xp[p - 1];
     // one entry at a time: sum over the (term, half) pairs that land on it
@@ -110,7 +112,7 @@ __device__ __forceinline__ void een_tables(const double *c, T x, T *tab)
     for (int d = 0; d <= D; d++)
 #pragma unroll
         for (int e = 0; e < NA; e++) {
-            T v = T(0);
+            C v = C(0);
 #pragma unroll
             for (int t = 0; t < ET.n; t++)
 #pragma unroll
@@ -118,10 +120,10 @@ __device__ __forceinline__ void een_tables(const double *c, T x, T *tab)
                     const int n = h == 0 ? ET.m[t] : ET.l[t] + ET.m[t];
                     const int p = h == 0 ? ET.l[t] + ET.m[t] : ET.m[t];
                     if (ET.idx[ET.k[t]][n] != e || p < d) continue;
-                    const T f = d == 0 ? T(1) : (d == 1 ? (T)p : (T)(p * (p - 1)));
-                    v += (T)c[t] * f * xp[p - d];
+                    const C f = d == 0 ? C(1) : (d == 1 ? (C)p : (C)(p * (p - 1)));
+                    v += (C)c[t] * f * xp[p - d];
                 }
-            tab[d * NA + e] = v;
+            tab[d * NA + e] = (T)v;
         }
 }
 

@@ -41,8 +41,10 @@ __global__ void __launch_bounds__(256) k_drift_old(MoveArgs a)
 // The sweeps of one determinant take k_sweep (engine_sweep.hip) instead.
 // A wavefront per 64 partners instead of one per walker: 256 electrons x 384
 // walkers 188 -> 73 us.
-#ifndef CHAMP_MOVE_WPE  // waves per SIMD asked of the register allocator
-#define CHAMP_MOVE_WPE 1
+// Waves per SIMD asked of the register allocator: four at order 5 on the FP32 path, which
+// misses them by five registers (97 electrons x 2048 walkers 49 us, with three 60).
+#ifndef CHAMP_MOVE_WPE
+#define CHAMP_MOVE_WPE (NORDC == 5 && sizeof(T) == sizeof(float) ? 4 : 1)
 #endif
 
 template <int NORDC, typename T>

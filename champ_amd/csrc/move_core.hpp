@@ -77,7 +77,7 @@ __device__ __forceinline__ void move_centres(const MoveGeo &g, const MoveLds<N, 
         L.rv[3 * c] = rv0; L.rv[3 * c + 1] = rv1; L.rv[3 * c + 2] = rv2;
         rnew[c] = r;
         rrnew[c] = rr;
-        if constexpr (N > 1) een_tables<N, 1, T>(jp.c[g.iwctype[c]], (T)(1.0 - kap * rr), L.tab + (size_t)c * 2 * een_naz<N>());
+        if constexpr (N > 1) een_tables<N, 1, T, double>(jp.c[g.iwctype[c]], 1.0 - kap * rr, L.tab + (size_t)c * 2 * een_naz<N>());
         if (rr != asymp_r) {
             const int it = g.iwctype[c];
             const double *a4 = jp.a4[it];
@@ -106,7 +106,12 @@ __device__ __forceinline__ void move_centres(const MoveGeo &g, const MoveLds<N, 
 // pair table (x, gradient factor; FP32, 8 bytes per pair instead of the two).
 // T: arithmetic type of the pair loop, the e-e-n tables and the AO values
 // (double on the FP64 path, float on the mixed path); distances of the moved
-// electron, the state and every sum across lanes stay double.
+// electron, the state and every sum across lanes stay double, and so does the e-e
+// value of a pair: its Pade constants are the same for all pairs, so an FP32 rounding
+// of one does not average out over the partners.  With them in FP32 the change of ln J
+// of a move against hpsi's FP64 pair sums (60 electrons) was off by -2.0e-6 in the mean,
+// 2.1e-6 rms; with the value and the tables (een_tables) formed in FP64 by 4e-10 and
+// 6e-8, in the same time (moves of 160 electrons x 4096 walkers 48.2 ms).
 template <int N, typename T>
 __device__ __forceinline__ void move_pair(const MoveGeo &g, const MoveLds<N, T> &L, const double *xw, double xn0,
                                           double xn1, double xn2, const double *rw, const double *rrw, const float2 *ew,
@@ -117,19 +122,30 @@ __device__ __forceinline__ void move_pair(const MoveGeo &g, const MoveLds<N, T> 
     const int NE = g.NE, NC = g.NC, iel = g.iel;
     const JasParams &jp = *g.jas;
     const double kap = jp.kap, asymp_r = jp.asymp_r;
-    const T tkap = (T)kap, tasymp = (T)asymp_r;
+    const T tkap = (T)kap;
     const int jq = j < NE ? j : 0;
     T fs = 0, sfu = 0, gm[3] = {0, 0, 0}, go[3] = {0, 0, 0};
     const double xd0 = xw[jq], xd1 = xw[NE + jq], xd2 = xw[2 * NE + jq];
     const T xj[3] = {(T)xd0, (T)xd1, (T)xd2};
     T dd1, fuf;
+    double fv = 0;  // FP32 path: the e-e value
     {
         const T rmo[3] = {(T)(xn0 - xd0), (T)(xn1 - xd1), (T)(xn2 - xd2)};
-        T r2 = 0;
-        r2 = r2 + rmo[0] * rmo[0]; r2 = r2 + rmo[1] * rmo[1]; r2 = r2 + rmo[2] * rmo[2];
-        const T rij = sqrt(r2);
-        const T u = scale_r<T>(tkap, rij);
-        dd1 = switched_from<T>(kap, rij, u);
+        T rij, u;
+        double ud = 0;
+        if constexpr (F32) {
+            double r2 = 0;
+            r2 = r2 + (xn0 - xd0) * (xn0 - xd0); r2 = r2 + (xn1 - xd1) * (xn1 - xd1); r2 = r2 + (xn2 - xd2) * (xn2 - xd2);
+            const double r = sqrt_inner(r2), x = exp_neg(-kap * r);
+            ud = (1.0 - x) * asymp_r;
+            rij = (T)r; dd1 = (T)x; u = (T)ud;
+        } else {
+            T r2 = 0;
+            r2 = r2 + rmo[0] * rmo[0]; r2 = r2 + rmo[1] * rmo[1]; r2 = r2 + rmo[2] * rmo[2];
+            rij = sqrt(r2);
+            u = scale_r<T>(tkap, rij);
+            dd1 = switched_from<T>(kap, rij, u);
+        }
         fuf = -tkap * dd1 / rij;
         // e-e term (jastrow4e.f90: psi_ee with its u-derivative)
         const int I = j > iel ? j : iel, J = j > iel ? iel : j;
@@ -139,23 +155,34 @@ __device__ __forceinline__ void move_pair(const MoveGeo &g, const MoveLds<N, T> 
             else if (jp.nocuspb == 0) sspinn = T(0.5);
             ipar = 1;
         }
-        if (on && (F32 || u != tasymp)) {
+        if (on && (F32 || u != (T)asymp_r)) {
             const double *b = jp.b[isb];
             T top = sspinn * (T)b[0] * u, topu = sspinn * (T)b[0];
             T bot = 1 + (T)b[1] * u, botu = (T)b[1], bot2 = bot * bot;
-            T fee = top / bot - (T)jp.jb[ipar];
             T feeu = topu / bot - botu * top / bot2;
-            T up = u;
-            for (int iord = 2; iord <= jp.nordb; iord++) {
-                T un = u * up;
-                fee = fee + (T)b[iord] * un;
-                feeu = feeu + (T)b[iord] * (T)iord * up;
-                up = un;
+            if constexpr (F32) {
+                fv = div_inner(sspinn * b[0] * ud, 1.0 + b[1] * ud) - jp.jb[ipar];
+                double upd = ud;
+                T up = u;
+                for (int iord = 2; iord <= jp.nordb; iord++) {
+                    feeu = feeu + (T)b[iord] * (T)iord * up;
+                    up = u * up;
+                    upd = ud * upd;
+                    fv = fv + b[iord] * upd;
+                }
+                feeu = feeu * dd1 / rij;
+            } else {
+                T fee = top / bot - (T)jp.jb[ipar];
+                T up = u;
+                for (int iord = 2; iord <= jp.nordb; iord++) {
+                    T un = u * up;
+                    fee = fee + (T)b[iord] * un;
+                    feeu = feeu + (T)b[iord] * (T)iord * up;
+                    up = un;
+                }
+                feeu = feeu * dd1 / rij;
+                fs += fee;
             }
-            feeu = feeu * dd1 / rij;
-            if constexpr (F32)  // value minus asymptote without cancellation
-                fee = pade_minus_asym<T>(b, jp.nordb, sspinn, u, asym_offset<T>(asymp_r, dd1), tasymp);
-            fs += fee;
             for (int k = 0; k < 3; k++) { gm[k] += feeu * rmo[k]; go[k] -= feeu * rmo[k]; }
         }
     }
@@ -214,7 +241,7 @@ __device__ __forceinline__ void move_pair(const MoveGeo &g, const MoveLds<N, T> 
     const T fu = sfu * fuf;
     const T rmo[3] = {(T)(xn0 - (double)xj[0]), (T)(xn1 - (double)xj[1]), (T)(xn2 - (double)xj[2])};
     for (int k = 0; k < 3; k++) { gi[k] = (double)(gm[k] + fu * rmo[k]); gj[k] = (double)(go[k] - fu * rmo[k]); }
-    f = (double)fs;
+    f = fv + (double)fs;
 }
 
 // R, R' of the radial instances tid, tid + nthr, ... at the moved electron

@@ -1,0 +1,38 @@
+"""Sums of the mixed path that two kernels form, one of them to subtract the other's:
+the pair sums of hpsi against those of the moves and of the quadrature."""
+import numpy as np
+import pytest
+
+from champ_amd import system as S
+from champ_amd.engine import PREC_FP64, PREC_MIXED, Engine
+from tests.gpu_helpers import ENGINE_LIB
+
+pytestmark = pytest.mark.gpu
+
+NWALK = 16 if "emu" in ENGINE_LIB else 64
+
+
+def molecule(nheavy, nh, nelec, order, ecp):
+    return S.make_system("sums", nheavy, nh, nelec, "ssppd", "sp", nloc=4 if ecp else 0, nordc=order)
+
+
+def change_of_ln_psi(sy, prec, x, moves):
+    eng = Engine(sy, len(x), precision=prec, lib_path=ENGINE_LIB)
+    eng.set_walkers(x)
+    psij = eng.hpsi()["psij"]
+    return np.array([eng.psie(i, xi)[1] - psij for i, xi in moves])
+
+
+@pytest.mark.parametrize("shape", [(9, 4, 60, 4, True), (5, 3, 33, 5, True), (5, 3, 33, 3, False)],
+                         ids=lambda s: "-".join(map(str, s)))
+def test_errors_of_a_moves_jastrow_scatter_about_zero(require_gpu, shape):
+    """ln J of a proposal minus that of hpsi: on the mixed path the roundings of the two
+    are independent from pair to pair, so their mean over n moves is within five standard
+    errors of 0; a constant rounded in one of them only shifts every pair the same way."""
+    sy = molecule(*shape)
+    x = sy.initial_walkers(NWALK, seed=21)
+    rng = np.random.default_rng(22)
+    moves = [(i, np.ascontiguousarray(x[:, i] + 0.3 * rng.standard_normal((NWALK, 3))))
+             for i in range(0, sy.nelec, sy.nelec // 8)]
+    d = change_of_ln_psi(sy, PREC_MIXED, x, moves) - change_of_ln_psi(sy, PREC_FP64, x, moves)
+    assert abs(d.mean()) < 5 * d.std() / np.sqrt(d.size), (d.mean(), d.std(), d.size)
