@@ -200,7 +200,7 @@ __global__ void __launch_bounds__(256) k_deriv_jastrow(DerArgs a)
                     double r2 = 0;
                     r2 = r2 + d0 * d0; r2 = r2 + d1 * d1; r2 = r2 + d2 * d2;
                     const double rij = sqrt(r2);
-                    const double u = switched_from<double>(kap, rij, scale_r(kap, rij));
+                    const double u = switched_from(kap, scale_r(kap, rij));
                     double up[NORDC + 1];
                     up[0] = 1.0;
 #pragma unroll

@@ -143,7 +143,7 @@ __global__ void __launch_bounds__(512) CHAMP_WAVES_PER_EU(CHAMP_HJAS_WPE) k_hpsi
                     ipar = 1;
                 }
                 const double u = scale_r(kap, rij);
-                const double dd1 = switched_from<double>(kap, rij, u), dd2 = -kap * dd1;
+                const double dd1 = switched_from(kap, u), dd2 = -kap * dd1;
                 uu1[s] = dd1;
                 dd1e[s] = -kap * dd1;
                 dd2e[s] = -kap * dd2;

@@ -25,41 +25,33 @@
 
 namespace champ {
 
-// psianl (nonlpsi.f90:88-105): e-n term at scaled distance rr; x = 1 - kap rr
-// (exp(-kap r)) for the float form, which subtracts the asymptote exactly
-template <typename T>
-__device__ __forceinline__ T en_term(const JasParams &jp, int it, T rr, T x)
+// psianl (nonlpsi.f90:88-105): e-n term at scaled distance rr
+__device__ __forceinline__ double en_term(const JasParams &jp, int it, double rr)
 {
-    if constexpr (sizeof(T) == sizeof(float))
-        return pade_minus_asym<T>(jp.a4[it], jp.norda, T(1), rr, asym_offset<T>(jp.asymp_r, x), (T)jp.asymp_r);
-    if (rr == (T)jp.asymp_r) return T(0);
-    T psi = (T)jp.a4[it][0] * rr / (T(1) + (T)jp.a4[it][1] * rr) - (T)jp.ja[it];
-    T rrip = rr;
-    for (int o = 2; o <= jp.norda; o++) { rrip = rrip * rr; psi = psi + (T)jp.a4[it][o] * rrip; }
+    if (rr == jp.asymp_r) return 0.0;
+    double psi = jp.a4[it][0] * rr / (1.0 + jp.a4[it][1] * rr) - jp.ja[it];
+    double rrip = rr;
+    for (int o = 2; o <= jp.norda; o++) { rrip = rrip * rr; psi = psi + jp.a4[it][o] * rrip; }
     return psi;
 }
 
-// psibnl (nonlpsi.f90:107-133): e-e term of electrons (i, j) at scaled u;
-// x = 1 - kap u (exp(-kap r)) for the float form
-template <typename T>
-__device__ __forceinline__ T ee_term(const JasParams &jp, int nup, int i, int j, T u, T x)
+// psibnl (nonlpsi.f90:107-133): e-e term of electrons (i, j) at scaled u
+__device__ __forceinline__ double ee_term(const JasParams &jp, int nup, int i, int j, double u)
 {
-    if (sizeof(T) != sizeof(float) && u == (T)jp.asymp_r) return T(0);
+    if (u == jp.asymp_r) return 0.0;
     const int I = j > i ? j : i, J = j > i ? i : j;
-    T sspinn = T(1);
+    double sspinn = 1.0;
     int isb = 0, ipar = 0;
     if (I < nup || J >= nup) {
         if (jp.nspin2b == 2) isb = 1;
-        else if (jp.nocuspb == 0) sspinn = T(0.5);
+        else if (jp.nocuspb == 0) sspinn = 0.5;
         ipar = 1;
     }
     const double *b = jp.b[isb];
-    if constexpr (sizeof(T) == sizeof(float))
-        return pade_minus_asym<T>(b, jp.nordb, sspinn, u, asym_offset<T>(jp.asymp_r, x), (T)jp.asymp_r);
-    const T fee = (T)b[0] * u / (T(1) + (T)b[1] * u);
-    T psi = sspinn * fee - (T)jp.jb[ipar];
-    T up = u;
-    for (int o = 2; o <= jp.nordb; o++) { up = u * up; psi = psi + (T)b[o] * up; }
+    const double fee = b[0] * u / (1.0 + b[1] * u);
+    double psi = sspinn * fee - jp.jb[ipar];
+    double up = u;
+    for (int o = 2; o <= jp.nordb; o++) { up = u * up; psi = psi + b[o] * up; }
     return psi;
 }
 
@@ -84,26 +76,25 @@ __device__ __forceinline__ double strided_sum(double v)
 constexpr int NL_THREADS = 256;
 constexpr int NL_WAVES = NL_THREADS / WAVE;
 
-// T: arithmetic type of the Jastrow part (double on the FP64 path, float on
-// the mixed path).  The determinant ratio at the points stays double on both
-// paths: sum_m phi_m W[i][m] cancels strongly when the inverse has large
-// entries, so FP32 AO values would lose its leading digits.  Sums across
-// lanes, the per-point assembly and every table in memory are double.
-template <int NORDC, int QB, typename T>
+// FP64 on both paths: it subtracts hpsi's pair sums (F, FP64 where a quadrature runs)
+// from its own at the points; in FP32 these would round their parameters, which adds up
+// over the partners (mixed path, 60 electrons, order 1: energies 6e-7 off their FP64
+// values in the median, 1.2e-5 rms over 300 walkers).  160 electrons x 1024 walkers:
+// 26.5 ms, in FP32 24.4; 60 electrons x 1000 walkers, order 1: 2.9 ms in either.
+template <int NORDC, int QB>
 __global__ void __launch_bounds__(NL_THREADS) CHAMP_WAVES_PER_EU(CHAMP_NL_WPE) k_nonloc(HArgs a)
 {
     HIP_DYNAMIC_SHARED(double, lds)
     const int tid = threadIdx.x, lane = tid % WAVE, wv = tid / WAVE;
     const int NE = a.NE, NC = a.NC, NQ = a.NQ, NB = a.NB, NRI = a.NRI;
     const JasParams &jp = *a.jas;
-    const T kap = (T)jp.kap, asymp = (T)jp.asymp_r;
-    const double kapd = jp.kap, asympd = jp.asymp_r;
+    const double kap = jp.kap, asymp = jp.asymp_r;
     double *S = lds;                        // [3][QB][NL_WAVES] per-wave sums: e-e, e-e-n + e-n, psi ratio
     double *XQ = S + 3 * QB * NL_WAVES;     // [QB][3] quadrature points
     double *FI = XQ + 3 * QB;               // [NL_WAVES] partial sums of F[i][.]
     double *GEO = FI + NL_WAVES;            // [QB][NC][5] point - centre: x, y, z, r, grid interval
     double *RAD = GEO + (size_t)QB * NC * 5;  // [QB][NRI] radial functions at the points
-    T *U = (T *)(RAD + (size_t)QB * NRI);   // [NE][QB] switched scaled e-e distances u(q, j)
+    double *U = RAD + (size_t)QB * NRI;     // [NE][QB] switched scaled e-e distances u(q, j)
 
     // XCD-aware assignment: workgroups are dealt round-robin to the 8 XCDs,
     // so the blocks b = x, x + 8, ... run on XCD x, which takes one contiguous
@@ -155,26 +146,26 @@ __global__ void __launch_bounds__(NL_THREADS) CHAMP_WAVES_PER_EU(CHAMP_NL_WPE) k
             {
                 const int qq = tid % QB;
                 const double px = XQ[3 * qq], py = XQ[3 * qq + 1], pz = XQ[3 * qq + 2];
-                T see = T(0);
+                double see = 0.0;
                 for (int j = tid / QB; j < NE; j += NL_THREADS / QB) {
-                    const T d0 = (T)(xw[j] - px), d1 = (T)(xw[NE + j] - py), d2 = (T)(xw[2 * NE + j] - pz);
-                    T r2 = 0;
+                    const double d0 = xw[j] - px, d1 = xw[NE + j] - py, d2 = xw[2 * NE + j] - pz;
+                    double r2 = 0;
                     r2 = r2 + d0 * d0; r2 = r2 + d1 * d1; r2 = r2 + d2 * d2;
-                    const T rjq = sqrt(r2);
-                    const T u = scale_r<T>(kap, rjq);
-                    const T xs = switched_from<T>(kapd, rjq, u);
+                    const double rjq = sqrt(r2);
+                    const double u = scale_r<double>(kap, rjq);
+                    const double xs = switched_from(kap, u);
                     U[(size_t)j * QB + qq] = xs;
-                    if (j != i) see += ee_term<T>(jp, a.NUP, i, j, u, xs);
+                    if (j != i) see += ee_term(jp, a.NUP, i, j, u);
                 }
-                const double sees = strided_sum<QB>((double)see);
+                const double sees = strided_sum<QB>(see);
                 if (lane < QB) S[(0 * QB + lane) * NL_WAVES + wv] = sees;
             }
             __syncthreads();
 
             // ---- phase B: e-e-n (lanes own a centre, stream over electrons) and e-n
-            T acc[QB];
+            double acc[QB];
 #pragma unroll
-            for (int qq = 0; qq < QB; qq++) acc[qq] = T(0);
+            for (int qq = 0; qq < QB; qq++) acc[qq] = 0.0;
             {
                 const int CT = NC < NL_THREADS ? NC : NL_THREADS, JG = NL_THREADS / CT;
                 for (int c0 = 0; c0 < NC; c0 += CT) {
@@ -182,30 +173,26 @@ __global__ void __launch_bounds__(NL_THREADS) CHAMP_WAVES_PER_EU(CHAMP_NL_WPE) k
                     if (jg < JG && c < NC) {
                         const int it = a.iwctype[c];
                         const double ecx = a.cent[3 * c], ecy = a.cent[3 * c + 1], ecz = a.cent[3 * c + 2];
-                        T A[QB][een_naz<NORDC>()];
+                        double A[QB][een_naz<NORDC>()];
                         bool any_asym = false;
                         bool asym[QB];
 #pragma unroll
                         for (int qq = 0; qq < QB; qq++) {
                             const double e0 = XQ[3 * qq] - ecx, e1 = XQ[3 * qq + 1] - ecy, e2 = XQ[3 * qq + 2] - ecz;
-                            if (jg == 0) {  // geometry of the point seen from centre c, for the AOs (double)
-                                double r2d = 0;
-                                r2d = r2d + e0 * e0; r2d = r2d + e1 * e1; r2d = r2d + e2 * e2;
-                                const double rqd = c == ic ? ren : sqrt(r2d);
+                            double r2 = 0;
+                            r2 = r2 + e0 * e0; r2 = r2 + e1 * e1; r2 = r2 + e2 * e2;
+                            const double rq = c == ic ? ren : sqrt(r2);
+                            if (jg == 0) {  // geometry of the point seen from centre c, for the AOs
                                 double *g = GEO + ((size_t)qq * NC + c) * 5;
-                                g[0] = e0; g[1] = e1; g[2] = e2; g[3] = rqd;
-                                g[4] = (double)grid_jx(a.tab, rqd);
+                                g[0] = e0; g[1] = e1; g[2] = e2; g[3] = rq;
+                                g[4] = (double)grid_jx(a.tab, rq);
                             }
-                            const T d0 = (T)e0, d1 = (T)e1, d2 = (T)e2;
-                            T r2 = 0;
-                            r2 = r2 + d0 * d0; r2 = r2 + d1 * d1; r2 = r2 + d2 * d2;
-                            const T rq = c == ic ? (T)ren : sqrt(r2);
-                            const T rr = scale_r<T>(kap, rq);
-                            const T xq = switched_from<T>(kapd, rq, rr);
+                            const double rr = scale_r<double>(kap, rq);
+                            const double xq = switched_from(kap, rr);
                             asym[qq] = rr == asymp;
                             any_asym = any_asym || asym[qq];
-                            if (jg == 0 && q0 + qq < NQ) acc[qq] += en_term<T>(jp, it, rr, xq);
-                            if constexpr (NORDC > 1) een_tables<NORDC, 0, T>(jp.c[it], xq, A[qq]);
+                            if (jg == 0 && q0 + qq < NQ) acc[qq] += en_term(jp, it, rr);
+                            if constexpr (NORDC > 1) een_tables<NORDC, 0>(jp.c[it], xq, A[qq]);
                         }
                         if constexpr (NORDC > 1) {
                             // one partner of lookahead on the scaled distance
@@ -214,15 +201,15 @@ __global__ void __launch_bounds__(NL_THREADS) CHAMP_WAVES_PER_EU(CHAMP_NL_WPE) k
                                 const double rrj = rr_next;
                                 if (j + JG < NE) rr_next = rrt[(size_t)(j + JG) * NC + c];
                                 if (j == i) continue;
-                                const T rj = (T)(1.0 - kapd * rrj);
-                                const T *uj = U + (size_t)j * QB;
-                                T P[QB];
+                                const double rj = 1.0 - kap * rrj;
+                                const double *uj = U + (size_t)j * QB;
+                                double P[QB];
 #pragma unroll
-                                for (int qq = 0; qq < QB; qq++) P[qq] = een_eval_tab<NORDC, 0, T>(A[qq], uj[qq], rj).f;
-                                if (any_asym && rrj == asympd) {  // psinl: both distances asymptotic -> 0
+                                for (int qq = 0; qq < QB; qq++) P[qq] = een_eval_tab<NORDC, 0>(A[qq], uj[qq], rj).f;
+                                if (any_asym && rrj == asymp) {  // psinl: both distances asymptotic -> 0
 #pragma unroll
                                     for (int qq = 0; qq < QB; qq++)
-                                        if (asym[qq]) P[qq] = T(0);
+                                        if (asym[qq]) P[qq] = 0.0;
                                 }
 #pragma unroll
                                 for (int qq = 0; qq < QB; qq++) acc[qq] += P[qq];
@@ -233,7 +220,7 @@ __global__ void __launch_bounds__(NL_THREADS) CHAMP_WAVES_PER_EU(CHAMP_NL_WPE) k
             }
 #pragma unroll
             for (int qq = 0; qq < QB; qq++) {
-                const double v = wave_sum((double)acc[qq]);
+                const double v = wave_sum(acc[qq]);
                 if (lane == 0) S[(1 * QB + qq) * NL_WAVES + wv] = v;
             }
 
@@ -350,9 +337,9 @@ template <> struct Mma<float> {
 // The e-e term minus its asymptote of the epilogue, per spin class (0 unlike,
 // 1 like) in a block's LDS: psi = p0 u / (1 + p1 u) - p2 + u^2 (p3 + u (p4 + ...)),
 // the coefficients past nordb zero.  The float form is (u - U)(p0 / (1 + p1 u)
-// + p2 + u (p3 + ...)), pade_minus_asym with its powers of the asymptote U
-// multiplied out (all of one sign pattern with the coefficients: nothing new
-// cancels).
+// + p2 + u (p3 + ...)) with u - U = -exp(-kap r) / kap for the distance to the
+// asymptote U = 1/kap and the powers of U multiplied out (all of one sign pattern
+// with the coefficients): near the asymptote nothing cancels.
 constexpr int EE_NP = CHAMP_NORDP + 1;
 template <typename T>
 __device__ __forceinline__ void ee_table(const JasParams &jp, T *tab)
@@ -384,7 +371,7 @@ __device__ __forceinline__ T ee_from_table(const T *p, T rr, T u, double asymp_r
         T g = p[EE_NP - 1];
 #pragma unroll
         for (int o = EE_NP - 2; o >= 2; o--) g = g * rr + p[o];
-        return asym_offset<T>(asymp_r, u) * (pade + g);
+        return (T)(-(double)u * asymp_r) * (pade + g);
     } else {
         T g = p[EE_NP - 1];
 #pragma unroll
@@ -621,7 +608,7 @@ __global__ void __launch_bounds__(MMA_THREADS) CHAMP_WAVES_PER_EU(CHAMP_MMA_WPE)
                         const double rq = b == ic ? a.r_en[((size_t)w * NC + ic) * NE + i] : sqrt_inner(r2);
                         xq = exp_neg(-kapd * rq);
                         const double rr = (1.0 - xq) * jp.asymp_r;
-                        sen += en_term<double>(jp, sT[b], rr, xq);
+                        sen += en_term(jp, sT[b], rr);
                         double xp[NORDC + 1];
                         een_powers<NORDC>(xq, xp);
                         een_uncoupled<NORDC>(jp.c[sT[b]], xp, sx);
@@ -945,41 +932,43 @@ static int launch_mma(champ_ctx *c, const HArgs &a)
     return CHAMP_OK;
 }
 
-template <int NORDC, int QB, typename T>
+template <int NORDC, int QB>
 static int launch_k(champ_ctx *c, const HArgs &a)
 {
-    const size_t lds = (3 * QB * NL_WAVES + 3 * QB + NL_WAVES + (size_t)QB * c->NC * 5 + (size_t)QB * c->NRI) * sizeof(double) +
-                       (size_t)c->NE * QB * sizeof(T);
+    const size_t lds = (3 * QB * NL_WAVES + 3 * QB + NL_WAVES + (size_t)QB * c->NC * 5 + (size_t)QB * c->NRI +
+                        (size_t)c->NE * QB) *
+                       sizeof(double);
+    if constexpr (QB > 2)  // fewer points at a time
+        if (lds > 160 * 1024) return launch_k<NORDC, 2>(c, a);
     if (lds > 160 * 1024) {
         set_error("nonloc: the quadrature kernel's LDS tables exceed 160 KB for this system");
         return CHAMP_ERR_UNSUPPORTED;
     }
     if (lds > 64 * 1024)
-        HIPCHECK(hipFuncSetAttribute((const void *)k_nonloc<NORDC, QB, T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        HIPCHECK(hipFuncSetAttribute((const void *)k_nonloc<NORDC, QB>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     // one wave of blocks: as many as can be resident at once
     int dev = 0, ncu = 256, per_cu = 1;
     HIPCHECK(hipGetDevice(&dev));
     HIPCHECK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-    HIPCHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_nonloc<NORDC, QB, T>, NL_THREADS, lds));
+    HIPCHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_nonloc<NORDC, QB>, NL_THREADS, lds));
     per_cu = std::max(1, per_cu);
     int slot;
     tbegin(c, K_HPSI_NONLOC, &slot);
-    hipLaunchKernelGGL((k_nonloc<NORDC, QB, T>), dim3(ncu * per_cu), dim3(NL_THREADS), lds, c->stream, a);
+    hipLaunchKernelGGL((k_nonloc<NORDC, QB>), dim3(ncu * per_cu), dim3(NL_THREADS), lds, c->stream, a);
     tend(c, slot);
     HIPCHECK(hipGetLastError());
     return CHAMP_OK;
 }
 
-template <typename T>
-static int launch_t(champ_ctx *c, const HArgs &a)
+static int launch_vector(champ_ctx *c, const HArgs &a)
 {
     switch (c->hjas.nordc) {
-    case 0: return launch_k<0, CHAMP_NL_QB, T>(c, a);
-    case 1: return launch_k<1, CHAMP_NL_QB, T>(c, a);
-    case 2: return launch_k<2, CHAMP_NL_QB, T>(c, a);
-    case 3: return launch_k<3, CHAMP_NL_QB, T>(c, a);
-    case 4: return launch_k<4, CHAMP_NL_QB, T>(c, a);
-    case 5: return launch_k<5, 2, T>(c, a);
+    case 0: return launch_k<0, CHAMP_NL_QB>(c, a);
+    case 1: return launch_k<1, CHAMP_NL_QB>(c, a);
+    case 2: return launch_k<2, CHAMP_NL_QB>(c, a);
+    case 3: return launch_k<3, CHAMP_NL_QB>(c, a);
+    case 4: return launch_k<4, CHAMP_NL_QB>(c, a);
+    case 5: return launch_k<5, 2>(c, a);
     default:
         set_error("nonloc: e-e-n order above 5 is not supported");
         return CHAMP_ERR_UNSUPPORTED;
@@ -1020,7 +1009,7 @@ int launch_nonloc(champ_ctx *c, const HArgs &a)
         default: return launch_mma<5, double>(c, a);
         }
     }
-    return c->prec == CHAMP_PREC_MIXED ? launch_t<float>(c, a) : launch_t<double>(c, a);
+    return launch_vector(c, a);
 }
 
 }  // namespace champ

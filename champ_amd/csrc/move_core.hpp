@@ -144,7 +144,7 @@ __device__ __forceinline__ void move_pair(const MoveGeo &g, const MoveLds<N, T> 
             r2 = r2 + rmo[0] * rmo[0]; r2 = r2 + rmo[1] * rmo[1]; r2 = r2 + rmo[2] * rmo[2];
             rij = sqrt(r2);
             u = scale_r<T>(tkap, rij);
-            dd1 = switched_from<T>(kap, rij, u);
+            dd1 = switched_from(kap, u);
         }
         fuf = -tkap * dd1 / rij;
         // e-e term (jastrow4e.f90: psi_ee with its u-derivative)

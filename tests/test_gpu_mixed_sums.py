@@ -36,3 +36,19 @@ def test_errors_of_a_moves_jastrow_scatter_about_zero(require_gpu, shape):
              for i in range(0, sy.nelec, sy.nelec // 8)]
     d = change_of_ln_psi(sy, PREC_MIXED, x, moves) - change_of_ln_psi(sy, PREC_FP64, x, moves)
     assert abs(d.mean()) < 5 * d.std() / np.sqrt(d.size), (d.mean(), d.std(), d.size)
+
+
+@pytest.mark.parametrize("order,form", [(1, -1), (4, 1)])
+def test_vector_pipe_quadrature_of_the_mixed_path(require_gpu, order, form):
+    """The vector-pipe quadrature subtracts hpsi's FP64 pair sums and forms its own the
+    same way: a mixed hpsi with it has no FP32 operation left, so the energies are those
+    of the FP64 path to the rounding of sums of a few thousand terms."""
+    sy = molecule(4, 3, 25, order, True)
+    x = sy.initial_walkers(8, seed=23)
+    e = {}
+    for prec in (PREC_FP64, PREC_MIXED):
+        eng = Engine(sy, len(x), precision=prec, lib_path=ENGINE_LIB)
+        eng.set_tuning(quadrature=form)
+        eng.set_walkers(x)
+        e[prec] = eng.hpsi()["energy"]
+    assert np.all(np.abs(e[PREC_MIXED] - e[PREC_FP64]) <= 1e-12 * np.maximum(1.0, np.abs(e[PREC_FP64])))
