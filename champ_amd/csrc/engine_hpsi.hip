@@ -18,17 +18,20 @@ namespace champ {
 #ifndef CHAMP_HJB
 #define CHAMP_HJB 1
 #endif
-#ifndef CHAMP_HJAS_WPE
-#define CHAMP_HJAS_WPE 1
+#ifndef CHAMP_HJAS_WPE  // FP32 at order 4: 128 registers instead of 143
+#define CHAMP_HJAS_WPE (NORDC == 4 && sizeof(T) == sizeof(float) ? 4 : 1)
 #endif
 constexpr int HJB = CHAMP_HJB;
 
-// FP64 on both paths: the mixed path's quadrature subtracts these pair sums from its
-// own at the points, and in FP32 the two round their parameters differently, which
-// adds up over the partners (energies of 512 walkers of 60 electrons 2e-6 to 4e-6 off
-// their FP64 values, 3e-7 to 4e-7 with these sums in FP64; of 160 electrons 5e-7 to
-// 9e-7, and 1e-7 to 2e-7).  160 electrons x 4096 walkers: 22.4 ms, in FP32 14.3.
-template <int NORDC>
+// T: arithmetic type of the pair loop.  FP32 on the mixed path of all-electron systems
+// (the e-e value and the e-e-n tables are formed in FP64 as in move_pair); FP64 where a
+// quadrature runs, which subtracts these sums from its own at the points: from FP32 sums,
+// energies of 512 walkers of 60 electrons were 2e-6 to 4e-6 off their FP64 values,
+// from FP64 sums 3e-7 to 4e-7 (of 160 electrons 5e-7 to 9e-7, and 1e-7 to 2e-7).
+// Distances, e-n terms and all sums over pairs are FP64 in both.
+// FP64: 160 electrons x 4096 walkers 22.4 ms; 176 electrons, 44 centres x 1024 walkers
+// 7.6 ms, in FP32 4.8 (5.8 at three waves per SIMD).
+template <int NORDC, typename T>
 __global__ void __launch_bounds__(512) CHAMP_WAVES_PER_EU(CHAMP_HJAS_WPE) k_hpsi_jastrow(HArgs a)
 {
     HIP_DYNAMIC_SHARED(double, lds)
@@ -94,78 +97,98 @@ __global__ void __launch_bounds__(512) CHAMP_WAVES_PER_EU(CHAMP_HJAS_WPE) k_hpsi
     // WAVE.  The row's per-centre e-e-n tables (value and two x-derivatives,
     // een_poly.hpp) and scalars are built by the wave into its LDS region.
     constexpr int NA = een_naz<NORDC>();
+    constexpr bool F32 = sizeof(T) == sizeof(float);
     constexpr int RS = 3 * NA + 8;  // doubles per centre: tables, r, rr, dd7, dd9, rvec (3), 1/r
     const int lane = tid % WAVE, wv = tid / WAVE, nwv = bd / WAVE;
-    double *rowt = lds + (size_t)wv * NC * RS;
+    T *rowt = (T *)lds + (size_t)wv * NC * RS;
+    const T tkap = (T)kap;
     for (int rr0 = wv; rr0 < NE - 1; rr0 += nwv) {
         const int i = NE - 1 - rr0;
         if constexpr (NORDC > 1) {
             __syncwarp();  // the previous row's table is no longer read
             for (int c = lane; c < NC; c += WAVE) {
-                double *rt = rowt + (size_t)c * RS;
+                T *rt = rowt + (size_t)c * RS;
                 const double ri = rw[(size_t)c * NE + i], rri = rrw[(size_t)c * NE + i];
-                const double sw = 1.0 - kap * rri;
-                een_tables<NORDC, 2>(jp.c[a.iwctype[c]], sw, rt);
-                rt[3 * NA] = ri;
-                rt[3 * NA + 1] = rri == asymp_r ? 1.0 : 0.0;  // electron i asymptotic for centre c
-                rt[3 * NA + 2] = -kap * sw;           // dd7
-                rt[3 * NA + 3] = -kap * (-kap * sw);  // dd9
-                for (int k = 0; k < 3; k++) rt[3 * NA + 4 + k] = xw[k * NE + i] - a.cent[3 * c + k];
-                rt[3 * NA + 7] = 1.0 / ri;
+                const T sw = (T)(1.0 - kap * rri);
+                een_tables<NORDC, 2, T, double>(jp.c[a.iwctype[c]], 1.0 - kap * rri, rt);
+                rt[3 * NA] = (T)ri;
+                rt[3 * NA + 1] = rri == asymp_r ? T(1) : T(0);  // electron i asymptotic for centre c
+                rt[3 * NA + 2] = -tkap * sw;           // dd7
+                rt[3 * NA + 3] = -tkap * (-tkap * sw);  // dd9
+                for (int k = 0; k < 3; k++) rt[3 * NA + 4 + k] = (T)(xw[k * NE + i] - a.cent[3 * c + k]);
+                rt[3 * NA + 7] = T(1) / (T)ri;
             }
             __syncwarp();
         }
         for (int j0 = 0; j0 < i; j0 += WAVE * HJB) {
-            double fs[HJB], d2[HJB], fI[HJB][3], fJ[HJB][3], rv[HJB][3], xj[HJB][3], sfu[HJB];
-            double uu1[HJB], dd1e[HJB], dd2e[HJB], irij[HJB], rij2[HJB];
+            T fs[HJB], d2[HJB], fI[HJB][3], fJ[HJB][3], rv[HJB][3], xj[HJB][3], sfu[HJB];
+            T uu1[HJB], dd1e[HJB], dd2e[HJB], irij[HJB], rij2[HJB];
+            double fv[HJB];  // FP32 form: the e-e value
             bool on[HJB];
 #pragma unroll
             for (int s = 0; s < HJB; s++) {
                 const int j = j0 + s * WAVE + lane;
                 on[s] = j < i;
                 const int jq = on[s] ? j : 0;
-                fs[s] = 0; d2[s] = 0; sfu[s] = 0;
+                fs[s] = 0; d2[s] = 0; sfu[s] = 0; fv[s] = 0;
                 for (int k = 0; k < 3; k++) {
                     fI[s][k] = 0; fJ[s][k] = 0;
                     const double xjd = xw[k * NE + jq];
-                    xj[s][k] = xjd;
-                    rv[s][k] = xw[k * NE + i] - xjd;
+                    xj[s][k] = (T)xjd;
+                    rv[s][k] = (T)(xw[k * NE + i] - xjd);
                 }
-                double r2 = 0;
-                r2 = r2 + rv[s][0] * rv[s][0]; r2 = r2 + rv[s][1] * rv[s][1]; r2 = r2 + rv[s][2] * rv[s][2];
-                const double rij = sqrt(r2);
+                T rij, u, dd1;
+                double ud = 0;
+                if constexpr (F32) {
+                    double r2 = 0;
+                    for (int k = 0; k < 3; k++) { const double d = xw[k * NE + i] - xw[k * NE + jq]; r2 = r2 + d * d; }
+                    const double r = sqrt_inner(r2), x = exp_neg(-kap * r);
+                    ud = (1.0 - x) * asymp_r;
+                    rij = (T)r; dd1 = (T)x; u = (T)ud;
+                } else {
+                    T r2 = 0;
+                    r2 = r2 + rv[s][0] * rv[s][0]; r2 = r2 + rv[s][1] * rv[s][1]; r2 = r2 + rv[s][2] * rv[s][2];
+                    rij = sqrt(r2);
+                    u = scale_r<T>(tkap, rij);
+                    dd1 = switched_from(kap, u);
+                }
                 rij2[s] = rij * rij;
-                irij[s] = 1.0 / rij;
-                double sspinn = 1; int isb = 0, ipar = 0;
+                irij[s] = T(1) / rij;
+                T sspinn = 1; int isb = 0, ipar = 0;
                 if (i < a.NUP || jq >= a.NUP) {
                     if (jp.nspin2b == 2) isb = 1;
-                    else if (jp.nocuspb == 0) sspinn = 0.5;
+                    else if (jp.nocuspb == 0) sspinn = T(0.5);
                     ipar = 1;
                 }
-                const double u = scale_r(kap, rij);
-                const double dd1 = switched_from(kap, u), dd2 = -kap * dd1;
+                const T dd2 = -tkap * dd1;
                 uu1[s] = dd1;
-                dd1e[s] = -kap * dd1;
-                dd2e[s] = -kap * dd2;
-                if (on[s] && u != asymp_r) {
+                dd1e[s] = -tkap * dd1;
+                dd2e[s] = -tkap * dd2;
+                if (on[s] && (F32 || u != (T)asymp_r)) {
                     const double *b = jp.b[isb];
-                    double top = sspinn * b[0] * u, topu = sspinn * b[0], topuu = 0;
-                    double bot = 1 + b[1] * u, botu = b[1], botuu = 0, bot2 = bot * bot;
-                    double fee = top / bot - jp.jb[ipar];
-                    double feeu = topu / bot - botu * top / bot2;
-                    double feeuu = topuu - (botuu * top + 2 * botu * topu) / bot + 2 * botu * botu * top / bot2;
+                    T top = sspinn * (T)b[0] * u, topu = sspinn * (T)b[0], topuu = 0;
+                    T bot = 1 + (T)b[1] * u, botu = (T)b[1], botuu = 0, bot2 = bot * bot;
+                    T fee = top / bot - (T)jp.jb[ipar];
+                    T feeu = topu / bot - botu * top / bot2;
+                    T feeuu = topuu - (botuu * top + 2 * botu * topu) / bot + 2 * botu * botu * top / bot2;
                     feeuu = feeuu / bot;
-                    double u1 = u, u2 = 1;  // uu(iord-1), uu(iord-2)
+                    T u1 = u, u2 = 1;  // uu(iord-1), uu(iord-2)
                     for (int iord = 2; iord <= jp.nordb; iord++) {
-                        const double un = u * u1;
-                        fee = fee + b[iord] * un;
-                        feeu = feeu + b[iord] * (double)iord * u1;
-                        feeuu = feeuu + b[iord] * (double)(iord * (iord - 1)) * u2;
+                        const T un = u * u1;
+                        fee = fee + (T)b[iord] * un;
+                        feeu = feeu + (T)b[iord] * (T)iord * u1;
+                        feeuu = feeuu + (T)b[iord] * (T)(iord * (iord - 1)) * u2;
                         u2 = u1; u1 = un;
                     }
                     feeuu = feeuu * dd1 * dd1 + feeu * dd2;
                     feeu = feeu * dd1 / rij;
-                    fs[s] += fee;
+                    if constexpr (F32) {  // the value in FP64
+                        fv[s] = div_inner(sspinn * b[0] * ud, 1.0 + b[1] * ud) - jp.jb[ipar];
+                        double up = ud;
+                        for (int iord = 2; iord <= jp.nordb; iord++) { up = ud * up; fv[s] = fv[s] + b[iord] * up; }
+                    } else {
+                        fs[s] += fee;
+                    }
                     for (int k = 0; k < 3; k++) { fI[s][k] += feeu * rv[s][k]; fJ[s][k] -= feeu * rv[s][k]; }
                     d2[s] += 2 * (feeuu + 2 * feeu);
                 }
@@ -183,11 +206,11 @@ __global__ void __launch_bounds__(512) CHAMP_WAVES_PER_EU(CHAMP_HJAS_WPE) k_hpsi
                     rrjn[s] = rrw[jcl[s]];
                 }
                 for (int c = 0; c < NC; c++) {
-                    const double *rt = rowt + (size_t)c * RS;
-                    const double ri = rt[3 * NA], dd7 = rt[3 * NA + 2], dd9 = rt[3 * NA + 3];
-                    const bool iasym = rt[3 * NA + 1] != 0.0;
-                    const double rvi0 = rt[3 * NA + 4], rvi1 = rt[3 * NA + 5], rvi2 = rt[3 * NA + 6], iri = rt[3 * NA + 7];
-                    const double cx = a.cent[3 * c], cy = a.cent[3 * c + 1], cz = a.cent[3 * c + 2];
+                    const T *rt = rowt + (size_t)c * RS;
+                    const T ri = rt[3 * NA], dd7 = rt[3 * NA + 2], dd9 = rt[3 * NA + 3];
+                    const bool iasym = rt[3 * NA + 1] != T(0);
+                    const T rvi0 = rt[3 * NA + 4], rvi1 = rt[3 * NA + 5], rvi2 = rt[3 * NA + 6], iri = rt[3 * NA + 7];
+                    const T cx = (T)a.cent[3 * c], cy = (T)a.cent[3 * c + 1], cz = (T)a.cent[3 * c + 2];
                     double rjc[HJB], rrjc[HJB];
 #pragma unroll
                     for (int s = 0; s < HJB; s++) {
@@ -201,22 +224,22 @@ __global__ void __launch_bounds__(512) CHAMP_WAVES_PER_EU(CHAMP_HJAS_WPE) k_hpsi
                     for (int s = 0; s < HJB; s++) {
                         if (j0 + s * WAVE >= i) break;
                         if (!on[s]) continue;
-                        const double rj = rjc[s];
+                        const T rj = (T)rjc[s];
                         if (iasym && rrjc[s] == asymp_r) continue;
-                        const double swj = 1.0 - kap * rrjc[s];
-                        const double dd8 = -kap * swj, dd10 = -kap * (-kap * swj);
-                        const EenOut<> e = een_eval_tab<NORDC, 2>(rt, uu1[s], swj);
-                        const double d1 = dd1e[s];
-                        const double fuu = e.fuu * d1 * d1 + e.fu * dd2e[s];
-                        const double fu = e.fu * d1 * irij[s];
-                        const double fui = e.fux * d1 * dd7, fuj = e.fuy * d1 * dd8;
-                        const double fii = e.fxx * dd7 * dd7 + e.fx * dd9, fjj = e.fyy * dd8 * dd8 + e.fy * dd10;
-                        const double irj = 1.0 / rj;
-                        const double fi = e.fx * dd7 * iri, fj = e.fy * dd8 * irj;
+                        const T swj = (T)(1.0 - kap * rrjc[s]);
+                        const T dd8 = -tkap * swj, dd10 = -tkap * (-tkap * swj);
+                        const EenOut<T> e = een_eval_tab<NORDC, 2, T>(rt, uu1[s], swj);
+                        const T d1 = dd1e[s];
+                        const T fuu = e.fuu * d1 * d1 + e.fu * dd2e[s];
+                        const T fu = e.fu * d1 * irij[s];
+                        const T fui = e.fux * d1 * dd7, fuj = e.fuy * d1 * dd8;
+                        const T fii = e.fxx * dd7 * dd7 + e.fx * dd9, fjj = e.fyy * dd8 * dd8 + e.fy * dd10;
+                        const T irj = T(1) / rj;
+                        const T fi = e.fx * dd7 * iri, fj = e.fy * dd8 * irj;
                         fs[s] += e.f;
                         sfu[s] += fu;
-                        const double st = (ri + rj) * (ri - rj);
-                        const double u2pst = rij2[s] + st, u2mst = rij2[s] - st;
+                        const T st = (ri + rj) * (ri - rj);
+                        const T u2pst = rij2[s] + st, u2mst = rij2[s] - st;
                         fI[s][0] += fi * rvi0; fI[s][1] += fi * rvi1; fI[s][2] += fi * rvi2;
                         fJ[s][0] += fj * (xj[s][0] - cx); fJ[s][1] += fj * (xj[s][1] - cy); fJ[s][2] += fj * (xj[s][2] - cz);
                         d2[s] = d2[s] + 2 * (fuu + 2 * fu) + fui * u2pst * (iri * irij[s]) + fuj * u2mst * (irj * irij[s]) + fii +
@@ -229,17 +252,17 @@ __global__ void __launch_bounds__(512) CHAMP_WAVES_PER_EU(CHAMP_HJAS_WPE) k_hpsi
                 const int j = j0 + s * WAVE + lane;
                 if (!on[s]) continue;
                 for (int k = 0; k < 3; k++) { fI[s][k] += sfu[s] * rv[s][k]; fJ[s][k] -= sfu[s] * rv[s][k]; }
-                const double fsd = fs[s];
+                const double fsd = fv[s] + (double)fs[s];
                 F[(size_t)i * NE + j] = fsd;
                 F[(size_t)j * NE + i] = fsd;
                 for (int k = 0; k < 3; k++) {
-                    const double gI = fI[s][k], gJ = fJ[s][k];
+                    const double gI = (double)fI[s][k], gJ = (double)fJ[s][k];
                     G1[((size_t)i * 3 + k) * NE + j] = gI;
                     G2[((size_t)i * 3 + k) * NE + j] = gJ;
                     G1[((size_t)j * 3 + k) * NE + i] = gJ;
                     G2[((size_t)j * 3 + k) * NE + i] = gI;
                 }
-                fsp += fsd; d2p += d2[s];
+                fsp += fsd; d2p += (double)d2[s];
             }
         }
     }
@@ -894,16 +917,17 @@ int launch_slater_refresh(champ_ctx *c)
     return CHAMP_OK;
 }
 
-static int launch_hpsi_jastrow(champ_ctx *c, const HArgs &a, int nordc, int naz)
+template <typename T>
+static int launch_hpsi_jastrow_t(champ_ctx *c, const HArgs &a, int nordc, int naz)
 {
     // up to 8 wavefronts per walker (one LDS row-table region each), so that
     // few walkers are in flight per XCD and their distance tables stay in L2
-    const size_t per_wave = nordc > 1 ? (size_t)c->NC * (3 * naz + 8) * sizeof(double) : 8;
+    const size_t per_wave = nordc > 1 ? (size_t)c->NC * (3 * naz + 8) * sizeof(T) : 8;
     const int nwv = (int)std::max<size_t>(1, std::min<size_t>(8, (160 * 1024 - 1024) / per_wave));
     const size_t lds = nwv * per_wave;
-    const void *fn = nordc == 5 ? (const void *)k_hpsi_jastrow<5> : nordc == 4 ? (const void *)k_hpsi_jastrow<4>
-                   : nordc == 3 ? (const void *)k_hpsi_jastrow<3> : nordc == 2 ? (const void *)k_hpsi_jastrow<2>
-                                                                            : (const void *)k_hpsi_jastrow<0>;
+    const void *fn = nordc == 5 ? (const void *)k_hpsi_jastrow<5, T> : nordc == 4 ? (const void *)k_hpsi_jastrow<4, T>
+                   : nordc == 3 ? (const void *)k_hpsi_jastrow<3, T> : nordc == 2 ? (const void *)k_hpsi_jastrow<2, T>
+                                                                            : (const void *)k_hpsi_jastrow<0, T>;
     if (lds > 160 * 1024) {
         set_error("hpsi: the Jastrow kernel's LDS tables exceed 160 KB for this system");
         return CHAMP_ERR_UNSUPPORTED;
@@ -911,11 +935,11 @@ static int launch_hpsi_jastrow(champ_ctx *c, const HArgs &a, int nordc, int naz)
     if (lds > 64 * 1024) HIPCHECK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     const dim3 block(WAVE * nwv);
     switch (nordc) {
-    case 5: hipLaunchKernelGGL(k_hpsi_jastrow<5>, dim3(c->W), block, lds, c->stream, a); break;
-    case 4: hipLaunchKernelGGL(k_hpsi_jastrow<4>, dim3(c->W), block, lds, c->stream, a); break;
-    case 3: hipLaunchKernelGGL(k_hpsi_jastrow<3>, dim3(c->W), block, lds, c->stream, a); break;
-    case 2: hipLaunchKernelGGL(k_hpsi_jastrow<2>, dim3(c->W), block, lds, c->stream, a); break;
-    default: hipLaunchKernelGGL(k_hpsi_jastrow<0>, dim3(c->W), block, lds, c->stream, a); break;
+    case 5: hipLaunchKernelGGL((k_hpsi_jastrow<5, T>), dim3(c->W), block, lds, c->stream, a); break;
+    case 4: hipLaunchKernelGGL((k_hpsi_jastrow<4, T>), dim3(c->W), block, lds, c->stream, a); break;
+    case 3: hipLaunchKernelGGL((k_hpsi_jastrow<3, T>), dim3(c->W), block, lds, c->stream, a); break;
+    case 2: hipLaunchKernelGGL((k_hpsi_jastrow<2, T>), dim3(c->W), block, lds, c->stream, a); break;
+    default: hipLaunchKernelGGL((k_hpsi_jastrow<0, T>), dim3(c->W), block, lds, c->stream, a); break;
     }
     HIPCHECK(hipGetLastError());
     return CHAMP_OK;
@@ -957,7 +981,9 @@ int launch_hpsi_impl(champ_ctx *c, int accumulate)
             set_error("hpsi: e-e-n order above 5 is not supported");
             return CHAMP_ERR_UNSUPPORTED;
         }
-        const int rcj = launch_hpsi_jastrow(c, a, nordc, naz[nordc]);
+        const bool f32 = c->prec == CHAMP_PREC_MIXED && c->nloc == 0;
+        const int rcj = f32 ? launch_hpsi_jastrow_t<float>(c, a, nordc, naz[nordc])
+                            : launch_hpsi_jastrow_t<double>(c, a, nordc, naz[nordc]);
         if (rcj) return rcj;
     }
     tend(c, slot);

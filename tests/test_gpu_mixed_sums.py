@@ -52,3 +52,22 @@ def test_vector_pipe_quadrature_of_the_mixed_path(require_gpu, order, form):
         eng.set_walkers(x)
         e[prec] = eng.hpsi()["energy"]
     assert np.all(np.abs(e[PREC_MIXED] - e[PREC_FP64]) <= 1e-12 * np.maximum(1.0, np.abs(e[PREC_FP64])))
+
+
+@pytest.mark.parametrize("shape", [(5, 3, 33, 5, False), (4, 4, 20, 4, False), (3, 1, 65, 1, False)],
+                         ids=lambda s: "-".join(map(str, s)))
+def test_pair_sums_without_a_quadrature_are_fp32(require_gpu, shape):
+    """An all-electron system has no quadrature that subtracts hpsi's pair sums: the
+    mixed path forms them in FP32 (their values differ from the FP64 ones), to the
+    rounding of FP32 terms."""
+    sy = molecule(*shape)
+    x = sy.initial_walkers(8, seed=24)
+    h = {}
+    for prec in (PREC_FP64, PREC_MIXED):
+        eng = Engine(sy, len(x), precision=prec, lib_path=ENGINE_LIB)
+        eng.set_walkers(x)
+        h[prec] = eng.hpsi()
+    for key, tol in (("psij", 2e-6), ("ekin", 2e-5)):
+        d = np.abs(h[PREC_MIXED][key] - h[PREC_FP64][key])
+        assert np.all(d <= tol * np.maximum(1.0, np.abs(h[PREC_FP64][key]))), key
+    assert np.any(h[PREC_MIXED]["ekin"] != h[PREC_FP64]["ekin"])
