@@ -28,7 +28,7 @@ FLAGS = [
     "-Wno-unused-result",
 ]
 # flags of single sources, with their reason in the source
-SOURCE_FLAGS = {"engine_sweep.hip": ["-mllvm", "-disable-machine-licm"]}
+SOURCE_FLAGS = {src: ["-mllvm", "-disable-machine-licm"] for src in ("engine_sweep.hip", "engine_nonloc.hip")}
 
 
 def _compile(src: str, objdir: str = OBJDIR, defines: tuple = ()) -> str:

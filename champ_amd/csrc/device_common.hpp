@@ -141,6 +141,12 @@ __device__ __forceinline__ T powi(T x, int m)
 #define CHAMP_WAVES_PER_EU(n) __attribute__((amdgpu_waves_per_eu(n)))
 #endif
 
+// A value that the compiler forms anew where this stands: what follows from the thread's
+// number is otherwise kept, or spilled, across a whole persistent loop.
+#ifndef FORM_AGAIN
+#define FORM_AGAIN(v) asm volatile("" : "+v"(v))
+#endif
+
 // four doubles / floats: the accumulator operands of the FP64 / FP32 MFMA instructions
 #ifndef CHAMP_DBL4_DEFINED
 typedef double dbl4 __attribute__((ext_vector_type(4)));

@@ -311,9 +311,15 @@ __global__ void __launch_bounds__(NL_THREADS) CHAMP_WAVES_PER_EU(CHAMP_NL_WPE) k
 // over the lanes once per group.
 // Bound: the epilogue (square root, exponential and Pade division per
 // (point, partner)) on the vector pipe, with the matrix cores beside it; three
-// waves per SIMD (168 registers) hide more of both than two.
-// Measured (160 electrons, 40 centres, 4096 walkers, about 1e7 points): 40.7 ms
-// with all entries in the product, 17.1 ms now; FP32 28.8 and 13.1 ms.
+// waves per SIMD (168 registers) hide more of both than two.  No form spills a
+// register: the thread's number is formed anew for each group and the lane's for each
+// item, and machine-level loop-invariant motion is off for this source (build.py);
+// else the addresses and constants of every phase stay live through all of them
+// (56 registers spilled in FP64 at order 4, 83 at order 5).
+// Measured (160 electrons, 40 centres, 4096 walkers): after ten sweeps (about 1e7
+// points) 40.7 ms with all entries in the product, 17.1 with the split; FP32 28.8 and
+// 13.1.  At the starting positions 13.9 ms with the spills, 13.2 without; FP32 10.9 and
+// 9.3.  97 electrons, order 5, 611 walkers: 1.18 and 1.02; FP32 0.83 and 0.67.
 constexpr int MMA_GP = NL_GROUP, MMA_MT = 3, MMA_MP = 16 * MMA_MT, MMA_THREADS = 256, MMA_WAVES = MMA_THREADS / WAVE;
 constexpr int MMA_TG = MMA_THREADS / MMA_MP;  // thread groups over (point, centre) in the point phase
 
@@ -393,7 +399,9 @@ __device__ __forceinline__ void mma_item(const HArgs &a, int w, int j0, int mt0,
     constexpr EenSplit<N> ES{};
     constexpr int NE_ = ES.nc > 0 ? ES.nc : 1, KC = ES.kmax > 0 ? ES.kmax : 1, NP = een_nsep<N>();
     typedef typename Mma<T>::acc Acc;
-    const int lane = threadIdx.x % WAVE, sl = lane / 16, ln = lane % 16;
+    int lane = threadIdx.x % WAVE;
+    FORM_AGAIN(lane);
+    const int sl = lane / 16, ln = lane % 16;
     const int NC = a.NC, NE = a.NE;
     const double kap = jp.kap;
     const int j = j0 + ln;
@@ -503,7 +511,6 @@ __global__ void __launch_bounds__(MMA_THREADS) CHAMP_WAVES_PER_EU(CHAMP_MMA_WPE)
     HIP_DYNAMIC_SHARED(double, lds)
     constexpr int NP = een_nsep<NORDC>();
     static_assert(MMA_GP * 12 <= MMA_MP, "group size");
-    const int tid = threadIdx.x, lane = tid % WAVE, wv = tid / WAVE;
     const int NE = a.NE, NC = a.NC, NQ = a.NQ, NC4 = (NC + 3) / 4 * 4;
     // the Jastrow parameters and the centres' types in LDS (read before use
     // behind the group loop's first barrier): every centre step of every item
@@ -511,9 +518,9 @@ __global__ void __launch_bounds__(MMA_THREADS) CHAMP_WAVES_PER_EU(CHAMP_MMA_WPE)
     __shared__ JasParams sJ;
     __shared__ int sT[128];
     static_assert(sizeof(JasParams) % 8 == 0, "JasParams copied as 8-byte words");
-    for (int t = tid; t < (int)(sizeof(JasParams) / 8); t += MMA_THREADS)
+    for (int t = threadIdx.x; t < (int)(sizeof(JasParams) / 8); t += MMA_THREADS)
         reinterpret_cast<unsigned long long *>(&sJ)[t] = reinterpret_cast<const unsigned long long *>(a.jas)[t];
-    for (int t = tid; t < NC; t += MMA_THREADS) sT[t] = a.iwctype[t];
+    for (int t = threadIdx.x; t < NC; t += MMA_THREADS) sT[t] = a.iwctype[t];
     __shared__ T sEE[2 * EE_NP];
     ee_table<T>(*a.jas, sEE);
     const JasParams &jp = sJ;
@@ -528,7 +535,7 @@ __global__ void __launch_bounds__(MMA_THREADS) CHAMP_WAVES_PER_EU(CHAMP_MMA_WPE)
     double *XK = FI + MMA_GP + MMA_MP + 2 * MMA_GP;            // [NP][MP] X_k of each point
     double *D0 = XK + NP * MMA_MP;                             // [GP][NP][NC] sum_j C_0n(y_jb) - C_0n(y_ib)
     T *XQ = (T *)(D0 + (size_t)MMA_GP * NP * NC);              // [NC4][MP] switched point-centre distances
-    for (int t = NC * MMA_MP + tid; t < NC4 * MMA_MP; t += MMA_THREADS) XQ[t] = T(0);
+    for (int t = NC * MMA_MP + threadIdx.x; t < NC4 * MMA_MP; t += MMA_THREADS) XQ[t] = T(0);
 
     const int G = gridDim.x, bk = blockIdx.x;
     const int nx = (G % 8 == 0) ? 8 : 1, gx = G / nx, xcd = bk % nx, g0 = bk / nx;
@@ -537,6 +544,9 @@ __global__ void __launch_bounds__(MMA_THREADS) CHAMP_WAVES_PER_EU(CHAMP_MMA_WPE)
     const int x_lo = xcd * per_x, x_hi = min(total, x_lo + per_x);
 
     for (int gi = x_lo + g0; gi < x_hi; gi += gx) {
+        int tid = threadIdx.x;
+        FORM_AGAIN(tid);
+        const int lane = tid % WAVE, wv = __builtin_amdgcn_readfirstlane(tid / WAVE);
         int lo = 0, hi = a.W - 1;
         while (lo < hi) {  // walker: largest w with grp_off[w] <= gi
             const int mid = (lo + hi + 1) / 2;

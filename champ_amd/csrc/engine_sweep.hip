@@ -29,11 +29,6 @@ __device__ __forceinline__ const MoveArgs &move_args_again()
     return *(const MoveArgs *)p;
 }
 #define MOVE_ARGS_AGAIN(a) move_args_again()
-// a value that the compiler forms anew at each use: what follows from the
-// thread's number would otherwise be kept across the whole sweep
-#define SWEEP_AGAIN(v) asm volatile("" : "+v"(v))
-#else
-#define SWEEP_AGAIN(v) (void)(v)
 #endif
 
 // What every move of every walker reads, in the block's LDS: the Jastrow
@@ -268,7 +263,7 @@ __global__ void __launch_bounds__(SW_BLOCK) CHAMP_WAVES_PER_EU(CHAMP_SWEEP_WPE) 
         // what follows from them would take more registers than there are
         const MoveArgs &a = MOVE_ARGS_AGAIN(args);
         int bt = threadIdx.x;
-        SWEEP_AGAIN(bt);
+        FORM_AGAIN(bt);
         const int wb = bt / NT, tid = bt % NT, wv = tid / WAVE, lane = tid % WAVE, w = blockIdx.x * wpb + wb;
         const bool live = w < a.W;  // a wavefront past the last walker only shares the block's tiles
         const int NE = a.NE, NC = a.NC, NO = a.NO, NM = a.NM, npad = SL::npad(NM);

@@ -18,6 +18,7 @@
 
 #define __global__
 #define MOVE_ARGS_AGAIN(a) (a)  // no kernel argument segment here
+#define FORM_AGAIN(v) (void)(v)  // nor vector registers to save
 #define __device__
 #define __host__
 #define __forceinline__ inline

@@ -122,3 +122,24 @@ def test_sweep_of_odd_shapes(require_gpu, shape, nwalk, mover):
         assert np.max(np.abs(got[w] - o.get_x())) < 1e-8
         assert abs(sc["psijo"][w] - d["psijo"]) < 1e-8 * max(1.0, abs(d["psijo"]))
         assert abs(sc["eold"][w] - d["eold"]) < 1e-6 * max(1.0, abs(d["eold"]))
+
+
+@pytest.mark.parametrize("prec", [PREC_FP64, PREC_MIXED])
+@pytest.mark.parametrize("order", [4, 5])
+def test_quadrature_forms_agree(require_gpu, order, prec):
+    """The matrix-core form against the vector-pipe form at several partner tiles, centre
+    steps and resident blocks: 97 electrons, 20 centres, 40 walkers."""
+    if "emu" in ENGINE_LIB:
+        pytest.skip("population too large for the host emulation")
+    sy = molecule(13, 7, 97, order, True)
+    x = sy.initial_walkers(40, seed=12)
+    e = []
+    for form, p in ((0, prec), (1, PREC_FP64)):
+        eng = Engine(sy, len(x), precision=p, lib_path=ENGINE_LIB)
+        eng.set_tuning(quadrature=form)
+        eng.set_walkers(x)
+        h = eng.hpsi()
+        e.append(h["energy"])
+    # FP64: the rounding of sums of a few thousand terms; mixed: FP32 terms summed in FP64
+    tol = 1e-9 if prec == PREC_FP64 else 2e-5
+    assert np.all(np.abs(e[0] - e[1]) <= tol * np.maximum(1.0, np.maximum(np.abs(e[1]), np.abs(h["ekin"]))))
