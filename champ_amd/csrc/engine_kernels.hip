@@ -29,8 +29,8 @@ __global__ void __launch_bounds__(256) k_drift_old(MoveArgs a)
 }
 
 // ------------------------------------------------------------------------
-// Move kernel A, one block per walker with a wavefront per 64 partner electrons
-// (at most four):
+// Move kernel A, a wavefront per 64 partner electrons of a walker (at most four; BLOCK)
+// or one wavefront per walker:
 //   mode 0: proposal from the drift at the old position: metrop1 (3 gauss
 //           draws; metrop_mov1_driftdif.f90:105-117) or metrop6 (local
 //           spherical move about the nearest nucleus; metrop6.hpp);
@@ -40,23 +40,28 @@ __global__ void __launch_bounds__(256) k_drift_old(MoveArgs a)
 //   writing the AO block that the MO GEMM contracts (orbitalse).
 // The sweeps of one determinant take k_sweep (engine_sweep.hip) instead.
 // A wavefront per 64 partners instead of one per walker: 256 electrons x 384
-// walkers 188 -> 73 us.
+// walkers 188 -> 73 us.  Up to 64 electrons a walker has one wavefront, without the
+// block's barriers, and above 512 walkers four of them share a block (launch_move_a_n).
 // Waves per SIMD asked of the register allocator: four at order 5 on the FP32 path, which
 // misses them by five registers (97 electrons x 2048 walkers 49 us, with three 60).
 #ifndef CHAMP_MOVE_WPE
 #define CHAMP_MOVE_WPE (NORDC == 5 && sizeof(T) == sizeof(float) ? 4 : 1)
 #endif
 
-template <int NORDC, typename T>
+template <int NORDC, typename T, bool BLOCK>
 __global__ void __launch_bounds__(256) CHAMP_WAVES_PER_EU(CHAMP_MOVE_WPE) k_move_a(MoveArgs a)
 {
     HIP_DYNAMIC_SHARED(double, lds)
-    const int wv = threadIdx.x / WAVE, lane = threadIdx.x % WAVE, nwv = blockDim.x / WAVE, w = blockIdx.x;
+    const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE, wv = BLOCK ? wave : 0;
+    const int nthr = BLOCK ? blockDim.x : WAVE, nwv = nthr / WAVE, tid = BLOCK ? threadIdx.x : lane;
+    const int w = BLOCK ? blockIdx.x : blockIdx.x * (blockDim.x / WAVE) + wave;
+    if (!BLOCK && w >= a.W) return;
     const int NE = a.NE, NC = a.NC, iel = a.iel;
-    const MoveLds<NORDC, T> L(lds, NC);
+    const size_t nlds = MoveLds<NORDC, T>::doubles(NC, a.NRI);
+    const MoveLds<NORDC, T> L(BLOCK ? lds : lds + wave * nlds, NC);
     // per 64 partners and lane: changes of the moved electron's sums [slot][4][WAVE]
-    double *Ldelta = lds + MoveLds<NORDC, T>::doubles(NC, a.NRI);
-    __shared__ double s_move[7];  // the proposal; the moved electron's e-n value and gradient
+    double *Ldelta = lds + nlds;  // BLOCK
+    __shared__ double s_move[3];  // the proposal
     const MoveGeo geo{NE, a.NUP, NC, iel, a.cent, a.iwctype, a.jas};
     const double *xw = a.xT + (size_t)w * 3 * NE;
     double xn0 = 0, xn1 = 0, xn2 = 0, en[4];
@@ -68,13 +73,10 @@ __global__ void __launch_bounds__(256) CHAMP_WAVES_PER_EU(CHAMP_MOVE_WPE) k_move
             xn0 = a.xnew[3 * w]; xn1 = a.xnew[3 * w + 1]; xn2 = a.xnew[3 * w + 2];
         }
         move_centres<NORDC, T>(geo, L, lane, xn0, xn1, xn2, a.rnew + (size_t)w * NC, a.rrnew + (size_t)w * NC, en);
-        if (lane == 0) {
-            s_move[0] = xn0; s_move[1] = xn1; s_move[2] = xn2;
-            for (int k = 0; k < 4; k++) s_move[3 + k] = en[k];
-        }
+        if (BLOCK && lane == 0) { s_move[0] = xn0; s_move[1] = xn1; s_move[2] = xn2; }
     }
-    __syncthreads();
-    xn0 = s_move[0]; xn1 = s_move[1]; xn2 = s_move[2];
+    team_sync<BLOCK>();
+    if (BLOCK) { xn0 = s_move[0]; xn1 = s_move[1]; xn2 = s_move[2]; }
     const double *fso_row = a.fso + ((size_t)w * NE + iel) * NE;
     const double *g1_row = a.g1 + ((size_t)w * NE + iel) * 3 * NE;
     const double *g2_row = a.g2 + ((size_t)w * NE + iel) * 3 * NE;
@@ -107,12 +109,16 @@ __global__ void __launch_bounds__(256) CHAMP_WAVES_PER_EU(CHAMP_MOVE_WPE) k_move
                 dj[1 + k] = gi[k] - g1_row[k * NE + j];
             }
         }
-        for (int k = 0; k < 4; k++) Ldelta[(size_t)(j0 / WAVE * 4 + k) * WAVE + lane] = dj[k];
+        if (BLOCK)
+            for (int k = 0; k < 4; k++) Ldelta[(size_t)(j0 / WAVE * 4 + k) * WAVE + lane] = dj[k];
+        else
+            for (int k = 0; k < 4; k++) d[k] += dj[k];
     }
-    __syncthreads();
+    team_sync<BLOCK>();
     if (wv == 0) {
-        for (int j0 = 0; j0 < NE; j0 += WAVE)  // in the order of the partners
-            for (int k = 0; k < 4; k++) d[k] += Ldelta[(size_t)(j0 / WAVE * 4 + k) * WAVE + lane];
+        if (BLOCK)
+            for (int j0 = 0; j0 < NE; j0 += WAVE)  // in the order of the partners
+                for (int k = 0; k < 4; k++) d[k] += Ldelta[(size_t)(j0 / WAVE * 4 + k) * WAVE + lane];
         for (int k = 0; k < 4; k++) d[k] = wave_sum(d[k]);
         if (lane == 0) {
             const double fsn_tot = a.fsumo[w] + d[0];
@@ -123,11 +129,11 @@ __global__ void __launch_bounds__(256) CHAMP_WAVES_PER_EU(CHAMP_MOVE_WPE) k_move
     }
     // ---- AOs of the moved electron (ider = 1) into the GEMM operand, as FP64, or
     // as FP32 for the FP32 contraction (a.ao32)
-    move_radial<NORDC, T>(L, threadIdx.x, blockDim.x, a.tab, a.NRI, a.ri_cent, a.ri_type, a.ri_rad, a.ri_rmax);
-    __syncthreads();
+    move_radial<NORDC, T>(L, tid, nthr, a.tab, a.NRI, a.ri_cent, a.ri_type, a.ri_rad, a.ri_rmax);
+    team_sync<BLOCK>();
     double *ao = a.aomove + (size_t)w * 4 * a.NB;
     float *ao32 = (float *)a.aomove + (size_t)w * 4 * a.NB;
-    for (int m = threadIdx.x; m < a.NB; m += blockDim.x) {
+    for (int m = tid; m < a.NB; m += nthr) {
         T out[5];
         move_ao(L, a.ao_cent[m], a.ao_ri[m], a.ao_slm[m], out);
         if (a.ao32) {
@@ -350,13 +356,28 @@ int launch_drift_old(champ_ctx *c, int iel)
     return CHAMP_OK;
 }
 
+#ifndef CHAMP_MOVE_PACK  // variant builds: walkers per block of single-wavefront walkers
+#define CHAMP_MOVE_PACK 0
+#endif
 template <int N, typename T>
 static int launch_move_a_n(champ_ctx *c, const MoveArgs &a)
 {
     const int slots = nblocks(c->NE, WAVE), nwv = std::min(4, slots);
-    const size_t lds = (MoveLds<N, T>::doubles(c->NC, c->NRI) + (size_t)slots * 4 * WAVE) * sizeof(double);
-    if (const int rc = move_lds((const void *)k_move_a<N, T>, lds)) return rc;
-    hipLaunchKernelGGL((k_move_a<N, T>), dim3(c->W), dim3(nwv * WAVE), lds, c->stream, a);
+    const size_t tables = MoveLds<N, T>::doubles(c->NC, c->NRI) * sizeof(double);
+    if (slots == 1) {
+        // up to 512 walkers a block each, so that they spread over the CUs.  us of the
+        // kernel with one / four walkers to a block: 60 electrons x 64 21.3 / 22.8, x 1024
+        // 28.1 / 27.3; 22 electrons x 512 22.2 / 24.0, x 2000 30.4 / 30.2 (mixed 31.8 / 28.8)
+        int wpb = CHAMP_MOVE_PACK ? CHAMP_MOVE_PACK : c->W <= 512 ? 1 : 4;
+        while (wpb > 1 && wpb * tables > MOVE_LDS_MAX) wpb /= 2;
+        const size_t lds = wpb * tables;
+        if (const int rc = move_lds((const void *)k_move_a<N, T, false>, lds)) return rc;
+        hipLaunchKernelGGL((k_move_a<N, T, false>), dim3(nblocks(c->W, wpb)), dim3(wpb * WAVE), lds, c->stream, a);
+    } else {
+        const size_t lds = tables + (size_t)slots * 4 * WAVE * sizeof(double);
+        if (const int rc = move_lds((const void *)k_move_a<N, T, true>, lds)) return rc;
+        hipLaunchKernelGGL((k_move_a<N, T, true>), dim3(c->W), dim3(nwv * WAVE), lds, c->stream, a);
+    }
     HIPCHECK(hipGetLastError());
     return CHAMP_OK;
 }

@@ -143,3 +143,26 @@ def test_quadrature_forms_agree(require_gpu, order, prec):
     # FP64: the rounding of sums of a few thousand terms; mixed: FP32 terms summed in FP64
     tol = 1e-9 if prec == PREC_FP64 else 2e-5
     assert np.all(np.abs(e[0] - e[1]) <= tol * np.maximum(1.0, np.maximum(np.abs(e[1]), np.abs(h["ekin"]))))
+
+
+# 9 and 64 electrons: one wavefront per walker, alone in its block or four to a block
+# (above 512 walkers; two where four walkers' tables of 120 centres would not fit);
+# 65: a wavefront per 64 partners
+@pytest.mark.parametrize("shape", [(2, 1, 9, 4, False), (6, 3, 64, 5, False), (100, 20, 64, 5, False), (6, 3, 65, 4, False)],
+                         ids=lambda s: "-".join(map(str, s)))
+@pytest.mark.parametrize("prec", [PREC_FP64, PREC_MIXED])
+def test_psie_does_not_depend_on_the_population(require_gpu, shape, prec):
+    """ln J and its gradient at a proposal, the same bits for a walker among 3 and among 517."""
+    if "emu" in ENGINE_LIB:
+        pytest.skip("population too large for the host emulation")
+    sy = molecule(*shape)
+    x = sy.initial_walkers(517, seed=14)
+    xn = x[:, 1] + 0.2
+    got = []
+    for part in (slice(0, 3), slice(0, 517)):
+        eng = Engine(sy, len(x[part]), precision=prec, lib_path=ENGINE_LIB)
+        eng.set_walkers(x[part])
+        eng.hpsi()
+        got.append((eng.psie(1, np.ascontiguousarray(xn[part]))[1], eng.array("vjn")))
+    for small, large in zip(*got):
+        assert np.array_equal(small, large[:3])
