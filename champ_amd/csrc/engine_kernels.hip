@@ -52,7 +52,8 @@ template <int NORDC, typename T, bool BLOCK>
 __global__ void __launch_bounds__(256) CHAMP_WAVES_PER_EU(CHAMP_MOVE_WPE) k_move_a(MoveArgs a)
 {
     HIP_DYNAMIC_SHARED(double, lds)
-    const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE, wv = BLOCK ? wave : 0;
+    const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const int wv = BLOCK ? wave : 0;
     const int nthr = BLOCK ? blockDim.x : WAVE, nwv = nthr / WAVE, tid = BLOCK ? threadIdx.x : lane;
     const int w = BLOCK ? blockIdx.x : blockIdx.x * (blockDim.x / WAVE) + wave;
     if (!BLOCK && w >= a.W) return;
@@ -366,8 +367,8 @@ static int launch_move_a_n(champ_ctx *c, const MoveArgs &a)
     const size_t tables = MoveLds<N, T>::doubles(c->NC, c->NRI) * sizeof(double);
     if (slots == 1) {
         // up to 512 walkers a block each, so that they spread over the CUs.  us of the
-        // kernel with one / four walkers to a block: 60 electrons x 64 21.3 / 22.8, x 1024
-        // 28.1 / 27.3; 22 electrons x 512 22.2 / 24.0, x 2000 30.4 / 30.2 (mixed 31.8 / 28.8)
+        // kernel with one / four walkers to a block: 60 electrons x 64 21.5 / 23.3, x 1024
+        // 27.9 / 27.6; 22 electrons x 512 22.7 / 24.5, x 2000 31.0 / 31.1 (mixed 32.6 / 30.3)
         int wpb = CHAMP_MOVE_PACK ? CHAMP_MOVE_PACK : c->W <= 512 ? 1 : 4;
         while (wpb > 1 && wpb * tables > MOVE_LDS_MAX) wpb /= 2;
         const size_t lds = wpb * tables;

@@ -246,7 +246,7 @@ __device__ __forceinline__ void sweep_orbitals(const MoveArgs &a, const MoveLds<
 // (mixed 72.9 -> 51.0), x 256 27.2 -> 8.4; 60 x 768 5.0 -> 2.2; 22 x 256 1.15 -> 0.49;
 // 10 x 4 0.41 -> 0.17.  Few walkers: the chains of one move (of 10 us at 10 electrons 4
 // are the proposal's and 3 the decision's scalar code); many: the pair loop, two waves
-// per SIMD of its 207 registers, on the FP64 pipe and on its 16 bytes per pair and centre.
+// per SIMD of its 227 registers (order 4), on the FP64 pipe and on its 16 bytes per pair and centre.
 template <int NORDC, typename T, int NW, int MOVERS>
 __global__ void __launch_bounds__(SW_BLOCK) CHAMP_WAVES_PER_EU(CHAMP_SWEEP_WPE) k_sweep(MoveArgs args, int e0, int e1)
 {
@@ -433,9 +433,11 @@ static inline int nblocks(int n, int per) { return (n + per - 1) / per; }
 // Threads per block of single-wavefront walkers.  Up to 512 walkers a block each, so
 // that they spread over the CUs; above, four share the coefficient reads and fill the
 // matrix instruction.  ms of a sweep's moves in blocks of one / four walkers:
-//   electrons 10, walkers 4     0.18 / 0.23    electrons 60, walkers 768  2.42 / 2.37
-//   22, 256                     0.53 / 0.58    160, 1024                  31.4 / 24.4
-//   60, 256                     2.06 / 2.07    160, 4096                  105.9 / 69.7
+//   electrons 10, walkers 4     0.18 / 0.22    electrons 97, walkers 520  6.90 / 5.75
+//   22, 256                     0.50 / 0.56    160, 520                   23.8 / 18.0
+//   60, 256                     1.89 / 2.03    160, 1024                  28.5 / 19.3
+//   60, 768                     2.19 / 2.24    160, 4096                  96.4 / 56.2
+//   60, 1000                    2.54 / 2.30
 static int one_wave_block(const champ_ctx *c)
 {
     if (CHAMP_SWEEP_BLOCK) return CHAMP_SWEEP_BLOCK;
@@ -446,10 +448,11 @@ static int one_wave_block(const champ_ctx *c)
 // resident at once (two on a CU, 512) and a move has the work for them, and where the
 // LDS of a block of single-wavefront walkers is too large; else one, which does
 // without barriers.  ms of a sweep's moves with one / four:
-//   electrons 10, walkers 4     0.18 / 0.18    electrons 160, walkers 256  22.2 / 10.0
-//   22, 256                     0.51 / 0.50    160, 1024                   24.4 / 23.3
-//   60, 256                     2.06 / 1.70    160, 4096                   69.7 / 91.9
-//   60, 768                     2.37 / 3.70
+//   electrons 10, walkers 4     0.18 / 0.18    electrons 97, walkers 520  5.75 / 6.80
+//   22, 256                     0.50 / 0.49    160, 256                   17.8 / 8.4
+//   60, 256                     1.89 / 1.62    160, 520                   18.0 / 17.4
+//   60, 520                     2.16 / 3.31    160, 1024                  19.3 / 20.2
+//   60, 768                     2.24 / 3.48    160, 4096                  56.2 / 79.1
 template <int N, typename T>
 static bool one_wave(const champ_ctx *c)
 {
