@@ -166,3 +166,79 @@ def test_psie_does_not_depend_on_the_population(require_gpu, shape, prec):
         got.append((eng.psie(1, np.ascontiguousarray(xn[part]))[1], eng.array("vjn")))
     for small, large in zip(*got):
         assert np.array_equal(small, large[:3])
+
+
+def sweep_against_oracle(sy, nwalk, walkers, lu_every=None, tau=0.3):
+    x = sy.initial_walkers(nwalk, seed=6)
+    eng = Engine(sy, nwalk, lib_path=ENGINE_LIB)
+    if lu_every is not None:
+        eng.set_lu_every(lu_every)
+    eng.set_walkers(x)
+    st = np.random.default_rng(5).integers(1, 2 ** 63 - 1, size=(nwalk, 4), dtype=np.uint64)
+    eng.set_rng(st)
+    eng.hpsi()
+    eng.metrop1(1, tau)
+    got, sc, rng = eng.get_walkers(), eng.scalars(), eng.get_rng()
+    for w in walkers:
+        o = ffi.walker(sy)
+        o.set_x(x[w])
+        o.set_rng(st[w])
+        if sy.nloc:
+            o.set_quad(sy.xq0, sy.yq0, sy.zq0)
+        o.hpsi()
+        o.sweep(tau)
+        d = o.scalars()
+        # as in test_sweep_of_odd_shapes
+        assert np.array_equal(rng[w], o.get_rng())
+        assert np.max(np.abs(got[w] - o.get_x())) < 1e-8
+        assert abs(sc["psijo"][w] - d["psijo"]) < 1e-8 * max(1.0, abs(d["psijo"]))
+        assert abs(sc["eold"][w] - d["eold"]) < 1e-6 * max(1.0, abs(d["eold"]))
+
+
+# spins of 132 and 131: a second pass over the orbitals beside ten columns of the update
+@pytest.mark.parametrize("nwalk", [2, 600])
+def test_sweep_of_large_spins(require_gpu, nwalk):
+    if "emu" in ENGINE_LIB:
+        pytest.skip("system too large for the host emulation")
+    sweep_against_oracle(molecule(40, 4, 263, 4, False), nwalk, (nwalk - 1,))
+
+
+# spins of 166 and 165: the update row by row.  Steps of 0.03 bohr: the determinant ratios
+# stay near 1, so that roundings add up and are not multiplied by small ratios' inverses
+@pytest.mark.parametrize("nwalk", [2, 600])
+def test_row_by_row_update(require_gpu, nwalk):
+    if "emu" in ENGINE_LIB:
+        pytest.skip("system too large for the host emulation")
+    sweep_against_oracle(molecule(40, 4, 331, 4, False), nwalk, (nwalk - 1,), tau=1e-3)
+
+
+@pytest.mark.parametrize("every", [1, 7, 32])
+def test_sweep_split_by_the_refresh(require_gpu, every):
+    """The inverse recomputed inside the sweep, every step but the last a whole one."""
+    sweep_against_oracle(molecule(5, 3, 33, 4, True), 3, (0, 2), lu_every=every)
+
+
+# 20 electrons: a walker per block, four to a block; 33 and 97: a block per walker,
+# then four walkers to a block (with a last block that is not full)
+@pytest.mark.parametrize("prec", [PREC_FP64, PREC_MIXED])
+@pytest.mark.parametrize("shape", [(4, 2, 20, 4, True), (5, 3, 33, 5, True), (13, 7, 97, 4, False)],
+                         ids=lambda s: "-".join(map(str, s)))
+def test_sweep_does_not_depend_on_the_population(require_gpu, shape, prec):
+    """The same bits for a walker among 3 and among 517."""
+    if "emu" in ENGINE_LIB:
+        pytest.skip("population too large for the host emulation")
+    sy = molecule(*shape)
+    x = sy.initial_walkers(517, seed=15)
+    st = np.random.default_rng(16).integers(1, 2 ** 63 - 1, size=(517, 4), dtype=np.uint64)
+    got = []
+    for n in (3, 517):
+        eng = Engine(sy, n, precision=prec, lib_path=ENGINE_LIB)
+        eng.set_tuning(orbital_gemm=0, ecp_rows_gemm=0 if sy.nloc else -1)  # hpsi's products too
+        eng.set_walkers(x[:n])
+        eng.set_rng(st[:n])
+        eng.hpsi()
+        eng.metrop1(2, 0.3)
+        sc = eng.scalars()
+        got.append((eng.get_walkers(), eng.get_rng(), sc["psijo"], sc["psido"]))
+    for small, large in zip(*got):
+        assert np.array_equal(small, large[:3])
