@@ -47,6 +47,7 @@ sys.path.insert(0, ROOT)
 #   hpsi_jastrow: Ne(Ne-1)/2 * Nc * (54T+80)
 #   hpsi_nonloc_psi (the psi ratio at each quadrature point, its own kernel):
 #       Nao*42 per point
+# Executed work of the sweep kernel's pair loop ("moves", k_sweep): flops_move_pairs.
 # Executed matrix-core work of the quadrature kernel (k_nonloc_mma): every
 # group of up to four active pairs of a walker runs, for each 16-partner tile,
 # each 16-point tile and each step of four centres, one 16x16x4 MFMA (2048
@@ -67,6 +68,30 @@ def een_ncoupled(nordc):
     term (k, l, m) with k, m >= 1 fills C[k][m] and C[k][l + m]."""
     from champ_amd import system as S
     return len({(k, n) for k, l, m in S.een_terms(nordc) if k >= 1 and m >= 1 for n in (m, l + m)})
+
+
+def een_eval_flops(nordc):
+    """Floating operations of een_poly.hpp's value and first derivatives at one
+    (pair, centre) from the tables (een_eval_tab, D = 1), counted over the same
+    Horner steps: a multiply-add is two."""
+    from champ_amd import system as S
+    nz = {(k, n) for k, l, m in S.een_terms(nordc) for n in (m, l + m)}
+    top = {k: max(n for kk, n in nz if kk == k) for k in {k for k, _ in nz}}
+    kmax, ops = max(top), 0
+    for k in range(kmax, -1, -1):
+        for n in range(top.get(k, 0) - 1, -1, -1):
+            ops += 2 if n < top[k] - 1 else 0              # d/dy: a copy at the row's first step
+            ops += 2 * (2 if (k, n) in nz else 1)          # value and d/dx rows
+        if k < kmax:
+            ops += 2 * (3 if k < kmax - 1 else 2) + 2      # P_u (a copy at the first step), P, P_y, P_x
+    return ops
+
+
+def flops_move_pairs(ne, nc, nordc, path):
+    """Executed floating operations of one move's pair loop (move_pair): the
+    polynomial and the two gradients per (partner, centre); FP32 reads the
+    partner's factors from a table that FP64 forms (two operations and a division more)."""
+    return (ne - 1) * nc * (een_eval_flops(nordc) + (19 if path == "mixed" else 23))
 
 
 def mfma_flops_nonloc(sy, nxq):
@@ -195,13 +220,13 @@ def run_hetero(args):
     return out
 
 
-# HBM bytes per launch of the matrix-core quadrature kernel (k_nonloc_mma,
-# the psi ratio excluded: it has its own kernel) at the default workload
-# (c160, 4096 walkers, the timed sweep after ten warm-up sweeps): FETCH_SIZE
-# x 2 + WRITE_SIZE x 1 from two rocprofv3 --pmc passes over the default bench,
-# scaled by the same counters on a device-to-device copy of known size
-# (profiles/k_nonloc_c160_traffic.md)
-NONLOC_TRAFFIC = {("c160", 4096, "fp64"): 1.29e9, ("c160", 4096, "mixed"): 1.20e9}
+# HBM bytes per launch of the sweep kernel (on the mixed path a launch is half a sweep)
+# and of the matrix-core quadrature kernel (the psi ratio has its own) at the default
+# workload (c160, 4096 walkers, after eleven sweeps): FETCH_SIZE x 2 + WRITE_SIZE x 1 from two
+# rocprofv3 --pmc passes, scaled by the same counters on a device-to-device copy of known
+# size (profiles/sweep_and_quadrature_c160_counters.md)
+TRAFFIC = {("moves", "c160", 4096, "fp64"): 1.38e11, ("moves", "c160", 4096, "mixed"): 4.95e10,
+           ("hpsi_nonloc", "c160", 4096, "fp64"): 1.44e9, ("hpsi_nonloc", "c160", 4096, "mixed"): 1.42e9}
 
 PEAK = {"fp64-mfma": 78.6, "fp32-mfma": 157.3, "fp64-valu": 78.6,
         # FP32 without packed math (this build never emits v_pk_* FP32): one
@@ -220,10 +245,12 @@ def per_kernel(sy, W, kt, nxq, path, acc):
     wchunk = W / -(-W // chunk)  # walkers per hpsi chunk launch, on average
     valu = "fp32-valu-unpacked" if path == "mixed" else "fp64-valu"
     mfma = "fp32-mfma" if path == "mixed" else "fp64-mfma"
+    # launches of a sweep: split where the inverse is recomputed
+    per_sweep = max(1.0, kt["moves"][1] / max(1, kt["hpsi_jastrow"][1])) if "moves" in kt and "hpsi_jastrow" in kt else 1.0
     work = {
-        "moves": (W * ne * (flops_move_jastrow(ne, nc, nt, nb, nrad) + 8.0 * ns * nb + acc * 4.0 * ns * ns), valu, "TFLOP/s",
-                  "reference count per move and walker: (Ne-1) Nc (25T+60) + AO, 8 Nsigma Nao, 4 Nsigma^2 per accepted",
-                  False),
+        "moves": (W * ne * flops_move_pairs(ne, nc, sy.nordc, path) / per_sweep, valu, "TFLOP/s",
+                  "executed operations of the pair loop per move and walker: (Ne-1) Nc (polynomial with first "
+                  "derivatives + gradients); the orbitals on the matrix cores and the inverse's update not counted", True),
         "move_jastrow_ao": (W * flops_move_jastrow(ne, nc, nt, nb, nrad), valu, "TFLOP/s",
                             "reference count (Ne-1) Nc (25T+60) + AO per walker", False),
         "move_mo_gemm": (2.0 * 4 * W * no * nb, "fp64-mfma", "TFLOP/s", "2 (4W) norb Nao", True),
@@ -261,17 +288,19 @@ def roofline(sy, W, kt, nxq, path, acc):
     pk = per_kernel(sy, W, kt, nxq, path, acc)
     dname = max((k for k in pk), key=lambda k: kt[k][0])
     d = pk[dname]
-    bound = "hbm" if d["pipe"] == "hbm" else "mfma"
+    bound = "hbm" if d["pipe"] == "hbm" else "mfma" if d["pipe"].endswith("mfma") else "valu"
+    traffic = TRAFFIC.get((dname, sy.name, W, path))
     r = {"bound": bound, "kernel": dname, "pipe": d["pipe"], "achieved": d["achieved"], "peak": d["peak"],
-         "unit": d["unit"], "frac": d["frac"], "traffic": None, "avg_launch_ms": d["avg_launch_ms"],
-         "work_per_launch": d["work_per_launch"], "work_basis": d["work_basis"]}
+         "unit": d["unit"], "frac": d["frac"], "utilisation": d["utilisation"], "traffic": traffic,
+         "traffic_source": "profiles/sweep_and_quadrature_c160_counters.md" if traffic else None,
+         "avg_launch_ms": d["avg_launch_ms"], "work_per_launch": d["work_per_launch"], "work_basis": d["work_basis"]}
+    if traffic:
+        r["traffic_GB_per_s"] = round(traffic / d["avg_launch_ms"] / 1e6, 1)
     if dname == "hpsi_nonloc":
         npts = float(np.sum(nxq))
         nt = len(S.een_terms(sy.nordc))
         ref = npts * flops_nonloc_point(sy.nelec, sy.ncent, nt, sy.nbasis)
         t = d["avg_launch_ms"] / 1e3
-        r["traffic"] = NONLOC_TRAFFIC.get((sy.name, W, path))
-        r["traffic_source"] = "profiles/k_nonloc_c160_traffic.md" if r["traffic"] else None
         r["quadrature_points_per_launch"] = int(npts)
         r["work_equivalent"] = {
             "achieved": round(ref / t / 1e12, 3), "unit": "TFLOP/s",
