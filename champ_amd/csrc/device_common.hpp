@@ -46,9 +46,10 @@ __device__ __forceinline__ double row16_sum(double v)
 // are ordinary distances: without the denormal scaling and the range checks
 // of the general functions, and with the polynomial of the exponential in
 // Estrin's form, which is half as long a chain as Horner's.  Newton and
-// Goldschmidt steps from the hardware estimates bring each to within an ulp
-// or two of the exact value (tests/cpu_emu/fastmath_check.cpp); 0 and infinity
-// give what the general functions give, NaN stays NaN.
+// Goldschmidt steps from the hardware estimates bring the root and the quotient
+// to within one ulp of the exact value, the exponential to within two
+// (tests/cpu_emu/inner_check.cpp).  0 and infinity give what the general root and
+// exponential give; a quotient needs a finite divisor other than 0.  NaN stays NaN.
 __device__ __forceinline__ double sqrt_inner(double x)
 {
     const double y = __builtin_amdgcn_rsq(x);
@@ -60,8 +61,9 @@ __device__ __forceinline__ double sqrt_inner(double x)
     g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
     return (x == 0.0 || x == __builtin_inf()) ? x : g;
 }
-// exp(x) for x <= 0: x = n ln 2 + f, the Taylor polynomial of degree 13 on
-// |f| <= ln 2 / 2 (remainder 4e-18)
+// exp(x) for x <= 0: x = n ln 2 + f with ln 2 in two parts after Cody and Waite (the
+// split of fdlibm's exp, whose high part times n is exact), the Taylor polynomial of
+// degree 13 on |f| <= ln 2 / 2 (remainder 4e-18)
 __device__ __forceinline__ double exp_neg(double x)
 {
     const double xc = x < -800.0 ? -800.0 : x;

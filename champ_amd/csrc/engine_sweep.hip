@@ -245,9 +245,9 @@ __device__ __forceinline__ void sweep_orbitals(const MoveArgs &a, const MoveLds<
 // product, decision and commit) and so: 160 electrons x 4096 walkers 90.3 -> 57.5
 // (mixed 72.9 -> 51.0), x 256 27.2 -> 8.4; 60 x 768 5.0 -> 2.2; 22 x 256 1.15 -> 0.49;
 // 10 x 4 0.41 -> 0.17.  Few walkers: the chains of one move (of 10 us at 10 electrons 4
-// are the proposal's and 3 the decision's scalar code); many: the pair loop, two waves
-// per SIMD of its 227 registers (order 4), on the FP64 pipe and on its 16 bytes per pair
-// and centre.
+// are the proposal's and 3 the decision's scalar code); many: memory latency, two waves
+// per SIMD (227 registers at order 4) waiting 62% of their cycles, with the vector pipe
+// 31% busy and 2.5 TB/s (16 bytes per pair and centre, and the commits) at 160 x 4096.
 template <int NORDC, typename T, int NW, int MOVERS>
 __global__ void __launch_bounds__(SW_BLOCK) CHAMP_WAVES_PER_EU(CHAMP_SWEEP_WPE) k_sweep(MoveArgs args, int e0, int e1)
 {

@@ -3,10 +3,12 @@
 // (jastrow4e.f90:3-358) and the radial functions and AOs (basis_fns.f90:8-214).
 //
 // Lanes take partner electrons, 64 at a time, and each pair's sum over the centres
-// is one chain on its lane; sums over partners are taken in their order.  So a
-// result does not depend on how many wavefronts share a walker or on which kernel
+// is one chain on its lane; sums over partners are taken in their order.  So ln J and
+// the AOs do not depend on how many wavefronts share a walker or on which kernel
 // asks: a trajectory amplifies roundings (a proposal with a small determinant
-// ratio by its inverse), and a sweep, psie and a forced move have to agree.
+// ratio by its inverse), and a sweep, psie and a forced move have to agree.  (Their
+// orbitals agree too with the tile form of the contraction in FP64; a tuned split-K or
+// FP32 contraction of psie rounds differently from the sweep, which has its own.)
 #pragma once
 #include "een_poly.hpp"
 #include "engine_internal.hpp"

@@ -416,7 +416,9 @@ class Engine:
         return dict(move_gemm=ch[0], orbital_gemm=ch[1], ecp_rows_gemm=ch[2], quadrature=ch[3])
 
     def set_tuning(self, move_gemm=-1, orbital_gemm=-1, ecp_rows_gemm=-1, quadrature=-1):
-        """Apply kernel choices without timing them (the layout autotune returns; -1: shape rule)."""
+        """Apply kernel choices without timing them (the layout autotune returns; -1: shape rule).
+        move_gemm is the contraction of psie, forced moves and multideterminant sweeps; a sweep of
+        one determinant has its own."""
         ch = (C.c_int32 * 4)(move_gemm, orbital_gemm, ecp_rows_gemm, quadrature)
         self._check(self.L.champ_gpu_set_tuning(self.ptr, ch), "set_tuning")
 

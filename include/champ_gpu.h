@@ -49,10 +49,14 @@ extern "C" {
 
 /* ---- precision modes ----------------------------------------------------- */
 #define CHAMP_PREC_FP64  0     /* every stage in IEEE double                      */
-/* FP32 arithmetic for AO values, the Jastrow (moves and hpsi) and the ECP
- * quadrature terms; FP64 for the AO->MO contraction (matrix cores), the
- * Sherman-Morrison updates, a full recompute of the Slater inverse every 80
- * moves, every sum across lanes and the local energy. */
+/* FP32 arithmetic for the AO values and the Jastrow pair terms of the moves
+ * (the e-e value and the e-e-n tables are formed in FP64), for the e-e and
+ * coupled e-e-n terms of the matrix-core ECP quadrature and, in all-electron
+ * systems, for hpsi's Jastrow pair terms; FP64 for hpsi's pair terms where a
+ * quadrature subtracts them, the quadrature's VALU form and psi ratio, the
+ * AO->MO contraction (matrix cores), the Sherman-Morrison updates, a full
+ * recompute of the Slater inverse every 80 moves, every sum across lanes and
+ * the local energy. */
 #define CHAMP_PREC_MIXED 1
 
 /*
@@ -438,14 +442,18 @@ int champ_gpu_metrop1_batch(champ_ctx *const *ctxs, int32_t n, int32_t nsweep,
  * 4: the tile form split over two halves of K with their partials added in a
  * fixed order, a candidate for the moves),
  * and the ECP quadrature form (0: matrix cores, 1: VALU); -1 where nothing was
- * tuned.  Leaves the walker state as
- * it was (hpsi is recomputed).  No counterpart in the reference.              */
+ * tuned.  "The moves" are psie, forced moves and the sweeps of
+ * multideterminant trial functions: a sweep of one determinant contracts its
+ * orbitals inside its own kernel, in FP64 on both paths, whatever the choice.
+ * Leaves the walker state as it was (hpsi is recomputed).  No counterpart in
+ * the reference.                                                              */
 int champ_gpu_autotune(champ_ctx *ctx, int32_t *choices);
 
 /* Applies kernel choices without timing them, in the layout autotune returns
  * (choices [4]; -1 restores the shape rule of that site).  GEMM kind 3 (FP32)
  * is accepted for the moves of the mixed path only, kind 4 (split K) for the
- * moves only.  No counterpart in the reference.                              */
+ * moves only; the choice for the moves does not reach the sweeps of one
+ * determinant (see champ_gpu_autotune).  No counterpart in the reference.    */
 int champ_gpu_set_tuning(champ_ctx *ctx, const int32_t *choices);
 
 /* on = 1: metrop1 replays each sweep as a HIP graph captured on first use

@@ -71,3 +71,19 @@ def test_pair_sums_without_a_quadrature_are_fp32(require_gpu, shape):
         d = np.abs(h[PREC_MIXED][key] - h[PREC_FP64][key])
         assert np.all(d <= tol * np.maximum(1.0, np.abs(h[PREC_FP64][key]))), key
     assert np.any(h[PREC_MIXED]["ekin"] != h[PREC_FP64]["ekin"])
+
+
+@pytest.mark.parametrize("shape", [(5, 3, 33, 5, True), (4, 4, 20, 4, True)], ids=lambda s: "-".join(map(str, s)))
+def test_pair_sums_under_a_quadrature_are_fp64(require_gpu, shape):
+    """With a pseudopotential hpsi's pair sums, orbitals and inverse are FP64 on both
+    paths: ln J and the kinetic energy agree to the rounding of sums of a few thousand terms."""
+    sy = molecule(*shape)
+    x = sy.initial_walkers(8, seed=25)
+    h = {}
+    for prec in (PREC_FP64, PREC_MIXED):
+        eng = Engine(sy, len(x), precision=prec, lib_path=ENGINE_LIB)
+        eng.set_walkers(x)
+        h[prec] = eng.hpsi()
+    for key in ("psij", "ekin"):
+        d = np.abs(h[PREC_MIXED][key] - h[PREC_FP64][key])
+        assert np.all(d <= 1e-12 * np.maximum(1.0, np.abs(h[PREC_FP64][key]))), key
